@@ -263,7 +263,9 @@ def selection_label(spb, A, mode, info, k):
     return f"learned (MLP pick {c.variant}{c.ipt}, measured neighbour kept: {form})"
 
 
-def kernel_name(info, k):
+def kernel_name(info, k, windowed=False):
+    if windowed:
+        return "k_spmv_win"
     if k > 1:
         return "k_spmv_mergeKg" if k >= 4 else "k_spmv_mergeK"
     if info.grid == -2:
@@ -332,10 +334,12 @@ def measure(spb, lib, name, args, variant=None, mode=None, steps=None, warmup=No
     graph_ms = graph_reps[2]
     log(f"{name}: wall {ms_step * 1e3:.1f} us/step  kernel {k_ms * 1e3:.1f} us  fixup "
         f"{fix_ms * 1e3:.1f} us  graph {graph_ms * 1e3:.1f} us")
-    traffic = stored_traffic(name, info)
+    # a chosen plan may run as windowed tiles in place of the kernel its shape names
+    windowed = bool(lib.vnec_plan_windowed(plan.h))
+    traffic = None if windowed else stored_traffic(name, info)
     rec = {
         "workload": desc, "nrows": m.nrows, "nnz": m.nnz, "nrhs": k,
-        "plan": {"variant": info.variant, "ipt": info.ipt, "grid": info.grid, "tiles": info.ntiles,
+        "plan": {"variant": info.variant, "ipt": info.ipt, "grid": info.grid, "tiles": info.ntiles, "windowed": windowed,
                  "selection": selection_label(spb, A, None if variant else mode, info, k)},
         "format_bytes": fb, "csr_bytes": B,
         "ms_per_step": round(ms_step, 5),
@@ -345,7 +349,7 @@ def measure(spb, lib, name, args, variant=None, mode=None, steps=None, warmup=No
                      "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(fb_main / (k_ms / 1e3) / 1e9 / HBM_PEAK_GBS, 4),
                      "traffic": traffic,
-                     "kernel": kernel_name(info, k), "kernel_us": round(k_ms * 1e3, 2),
+                     "kernel": kernel_name(info, k, windowed), "kernel_us": round(k_ms * 1e3, 2),
                      "fixup_us": round(fix_ms * 1e3, 2),
                      "algorithmic_bytes_per_launch": fb_main,
                      "csr_equivalent_GBps": round(B / (k_ms / 1e3) / 1e9, 1),

@@ -101,7 +101,11 @@ typedef enum {
 } vnec_encoding;
 
 /* Negative vnec_tuning.variant values: how the plan chooses its variant,
- * tile granularity and schedule. */
+ * tile granularity and schedule.  A plan the learned or autotune mode, an FP32
+ * selection or a Build_VNEC_* call chose runs as windowed tiles (distinct x
+ * entries of a tile gathered into LDS once) where those are the faster form of
+ * what it picked; vnec_plan_info_ext still reports the pick, with the windowed
+ * tiles' count. */
 typedef enum {
     VNEC_SELECT_LEARNED = -1,   /* the trained MLP over matrix statistics (the
                                    rule below when no model is installed)    */

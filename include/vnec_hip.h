@@ -207,6 +207,64 @@ int vnec_hip_tile_colspan(const int32_t *coords, int64_t ntiles, const int32_t *
 /* Whether a (variant, ipt, encoding, nrhs) combination is compiled in. */
 int vnec_hip_merge_supported(int variant, int ipt, int encoding, int nrhs);
 
+/* Windowed tiles (one right-hand side): tiles of at most VNEC_WIN_THREADS *
+ * ipt nonzeros whose distinct x entries are gathered into LDS once
+ * (vnec_win.hip).  Slots: tile t's nonzeros from t VNEC_WIN_THREADS ipt on,
+ * thread k holding nonzeros k ipt .. k ipt + ipt - 1 of the tile. */
+#define VNEC_WIN_THREADS 512
+#define VNEC_WIN_MAX_IPT 16 /* ipt: 4, 8 or 16                              */
+#define VNEC_WIN_ROWS 8     /* rows that weigh as much as a nonzero         */
+typedef struct {
+    const int32_t *desc;    /* 8 per tile: first row, first nonzero, rows
+                               ended, nonzeros, distinct columns, and of the
+                               row begun before the tile its first tile and
+                               tile count (0: none), of the row begun in and
+                               left unfinished by it its tile count (0: none) */
+    int64_t ntiles;
+    int entries;            /* LDS entries of the largest tile              */
+    const int32_t *win;     /* distinct columns, tile t's ascending from its
+                               first nonzero's index on; or, when woff is
+                               given, 16 bits each:                         */
+    const int32_t *wbase;   /* the first of every 64 and                    */
+    const uint16_t *woff;   /* each one's distance from it, tile t's from
+                               chunk (first nonzero >> 6) + t on            */
+    const double *wv;       /* slots: values (encoding FP64)                */
+    const float *whi, *wlo; /* slots: FP32 hi (+ lo), or FP32 values        */
+    const uint16_t *wl;     /* slots: rank of the column in the window      */
+    const uint32_t *wt;     /* per thread: row-end flags | ordinal of its
+                               first row end in the tile << 16              */
+    const uint64_t *rmask;  /* per tile and 64 of its rows, from word
+                               (first row >> 6) + t on: rows with nonzeros  */
+    const uint16_t *rbase;  /* in the tile, and the ordinal of the first    */
+    const double *x;
+    double *y;
+    double *slot;           /* ntiles: partial sums of cut rows, all empty
+                               between launches                             */
+    const float *x32;
+    float *y32;
+    float *slot32;
+    int ipt, encoding;
+} vnec_win_args;
+/* Tile boundaries (coords, 2 (P + 1) ints) every `step` units of nonzeros
+ * plus rows / VNEC_WIN_ROWS; step + snap <= VNEC_WIN_THREADS * ipt. */
+int vnec_hip_win_coords(const int32_t *ptr, int64_t nrows, int64_t nnz, int64_t P, int64_t step, int snap,
+                        int32_t *coords, void *stream);
+int vnec_hip_win_desc(const int32_t *ptr, int64_t nrows, const int32_t *coords, int64_t ntiles, const int32_t *nec,
+                      int32_t *desc, void *stream);
+/* wbase / woff from the windows uniq / nec of vnec_hip_ecr_tiles_pass1;
+ * *wide (caller-zeroed) is set when a distance does not fit 16 bits. */
+int vnec_hip_win_list(const int32_t *coords, int64_t ntiles, const int32_t *uniq, const int32_t *nec, int32_t *wbase,
+                      uint16_t *woff, int32_t *wide, void *stream);
+/* Slots, flags, masks, per-tile LDS entries (nsum) and their maximum
+ * (*max_dev, caller-zeroed); empties the slots of partial sums. */
+int vnec_hip_win_layout(const int32_t *ptr, const double *val, const uint16_t *lcol, const int32_t *coords,
+                        int64_t ntiles, int ipt, int encoding, double *wv, float *whi, float *wlo, uint16_t *wl,
+                        uint32_t *wt, uint64_t *rmask, uint16_t *rbase, const int32_t *nec, int32_t *nsum,
+                        int32_t *max_dev, void *slot, void *stream);
+/* Lets the kernel of these arguments use the LDS it needs (once per plan). */
+int vnec_hip_win_prepare(const vnec_win_args *a);
+int vnec_hip_spmv_win(const vnec_win_args *a, void *stream);
+
 /* Gather-ceiling probe over a matrix's values and columns (nnz): with
  * gather = 0 it streams them, with gather = 1 it also gathers x[col] per
  * nonzero; no row structure; out holds grid * 256 partial sums. */

@@ -1,0 +1,194 @@
+"""Windowed tiles (vnec_win.hip): what the learned mode, SpB_mxv and the
+Build_VNEC_* plans run in place of merge-path, block and slice kernels.
+
+Each matrix sits at an edge of the layout — a tile's end, a row cut by one or
+many tile boundaries, rows without nonzeros, windows too sparse for 16-bit
+lists, columns repeated or descending — and is checked per row against the
+oracle's long-double sums, |y - y_ref| <= tol (|A||x|)_i: 1e-12 for FP64 and hi
++ lo values, 2^-23 for hi-only, the FP32 API's row gate for FP32; against the
+general merge-path plan of the same matrix within twice that; and bit for bit
+over repeated and replayed launches."""
+import numpy as np
+import pytest
+
+import oracle as O
+from vnec_amd import matgen as g
+from vnec_amd import spb
+
+pytestmark = pytest.mark.gpu
+TOL = {"fp64": 1e-12, "hilo": 1e-12, "hi": 2.0 ** -23}
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _gpu():
+    if spb.device_count() < 1:
+        pytest.fail("no GPU visible: the gpu tests need an MI355X")
+    spb.init()
+
+
+def _windowed(p):
+    return bool(spb.L.load().vnec_plan_windowed(p.h))
+
+
+def _rows(lens, ncols, seed, cols=None):
+    """CSR of the given row lengths; columns random, ascending and distinct
+    within a row unless given."""
+    rng = np.random.default_rng(seed)
+    ptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    if cols is None:
+        cols = np.concatenate([np.sort(rng.choice(ncols, n, replace=False)) for n in lens] or [np.zeros(0)])
+    return g.from_pattern(len(lens), ncols, ptr, cols.astype(np.int32), seed=seed)
+
+
+def _tile_edge(n):  # n nonzeros in rows of one, then a last row of three
+    return _rows([1] * (n - 3) + [3], 4096, n)
+
+
+def _cut_rows():  # rows over 1, 2, 3, 5, 9 and 40 tiles of 2048, short and empty ones between
+    lens = []
+    for k in (1, 2, 3, 5, 9, 40):
+        lens += [0, 2, 2048 * k - 7, 1, 0, 0, 5]
+    return _rows(lens, 100000, 5)
+
+
+def _empty_stretches():
+    return _rows([0] * 5000 + [3, 0, 4] * 40 + [0] * 70000 + [64, 0, 1] + [0] * 3000, 2000, 6)
+
+
+def _sparse_window():  # 64 neighbouring window entries lie half a million columns apart
+    return _rows([3] * 400, 8_000_000, 7)
+
+
+def _repeated_descending():
+    rng = np.random.default_rng(8)
+    lens = rng.integers(0, 40, 3000)
+    return _rows(lens, 500, 8, cols=np.concatenate(
+        [np.sort(np.repeat(rng.integers(0, 500, n), 1))[::-1] for n in lens]))
+
+
+def _lds_limit():  # rows of one nonzero, then rows of six
+    rng = np.random.default_rng(13)
+    lens = np.repeat([1, 6], [300000, 220000])
+    return _rows(lens, 1 << 20, 13, cols=rng.integers(0, 1 << 20, int(lens.sum())))
+
+
+MATRICES = {
+    "one": lambda: _rows([1], 1, 1),
+    "edge2047": lambda: _tile_edge(2047), "edge2048": lambda: _tile_edge(2048), "edge2049": lambda: _tile_edge(2049),
+    "cut_rows": _cut_rows, "empty_stretches": _empty_stretches, "sparse_window": _sparse_window,
+    "repeated_descending": _repeated_descending,
+    "ipt8": lambda: g.powerlaw(60013, 2.2, 3, 20000, seed=9),   # 4096-item tiles, long rows
+    "ipt16": lambda: g.rmat(17, 12, seed=10),                   # 8192-item tiles
+    "short_rows": lambda: g.uniform(393241, 3, seed=11),        # as many row sums as window entries
+    "lds_limit": _lds_limit,                                    # 8192-item tiles would not leave room for two
+    "dense_row": lambda: g.skew(13, 80, 2, 8000, seed=12),
+}
+
+
+def _check(m, y, enc, ref=None):
+    if enc == "fp32":
+        v, x = m.val.astype(np.float32), m.x.astype(np.float32)
+        ax, _ = O.spmv_abs(m.ptr, m.col, v.astype(np.float64), x.astype(np.float64))
+        return O.check_rows_f32(y, O.spmv_serial_f32(m.ptr, m.col, v, x) if ref is None else ref, m.ptr, ax)
+    ax, yl = O.spmv_abs(m.ptr, m.col, m.val, m.x)
+    return O.check_rows(y, yl if ref is None else ref, ax, TOL[enc] * (1 if ref is None else 2))
+
+
+@pytest.mark.parametrize("enc", ["fp64", "hilo", "hi", "fp32"])
+@pytest.mark.parametrize("name", list(MATRICES))
+def test_windowed_plan_matches_oracle_and_general_plan(name, enc):
+    m = MATRICES[name]()
+    dt = np.float32 if enc == "fp32" else np.float64
+    print(f"windowed {name} {enc}: {m.nrows} x {m.ncols}, {m.nnz} nonzeros", flush=True)
+    A = spb.Matrix.from_csr(m.nrows, m.ncols, m.ptr, m.col, m.val.astype(dt), dtype=dt)
+    p = spb.Plan(A, "learned", encoding=enc)
+    if p.info().variant == "G":
+        pytest.fail("a pattern matrix: not what this test is for")
+    assert _windowed(p), p.info()
+    q = spb.Plan(A, "L", 7, encoding=enc, grid=-1)  # a named shape keeps its kernel
+    assert not _windowed(q)
+    dx = spb.DeviceArray.from_array(m.x.astype(dt))
+    ys = []
+    for run in (p.spmv_dev, p.spmv_dev, p.spmv_graph, p.spmv_graph, q.spmv_dev):
+        dy = spb.DeviceArray.from_array(np.full(m.nrows, np.nan, dt))
+        run(dx.ptr, dy.ptr)
+        ys.append(dy.to_array(dt, m.nrows))
+        dy.free()
+    for y in ys[1:4]:
+        assert np.array_equal(y.view(np.uint8), ys[0].view(np.uint8)), "repeated SpMV changed bits"
+    ok, worst = _check(m, ys[0], enc)
+    assert ok, worst
+    ok, worst = _check(m, ys[0], enc, ref=ys[4])
+    assert ok, worst
+    fb, _ = p.format_bytes()
+    assert fb >= (4 if enc in ("hi", "fp32") else 8) * m.nnz
+    for h in (p, q):
+        h.free()
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+def test_windowed_infinities_and_nan_stay_in_their_rows(dt):
+    """x entries of +Inf, -Inf and NaN reach exactly the rows that hold their
+    columns — not the slots a tile leaves unused, nor the next launch through
+    the partial sums of rows that many tiles share — and the sums agree with
+    the general plan's class by class."""
+    m = _cut_rows()
+    A = spb.Matrix.from_csr(m.nrows, m.ncols, m.ptr, m.col, m.val.astype(dt), dtype=dt)
+    p, q = spb.Plan(A, "learned"), spb.Plan(A, "L", 7, grid=-1)
+    assert _windowed(p)
+    long_row = int(np.argmax(np.diff(m.ptr)))
+    lo = int(m.ptr[long_row])
+    clean = m.x.astype(dt)
+    want = None
+    for bad in ({}, {m.col[lo]: np.inf}, {m.col[lo]: np.nan, m.col[lo + 5000]: -np.inf, 0: np.inf}, {}):
+        x = clean.copy()
+        for c, v in bad.items():
+            x[c] = v
+        dx = spb.DeviceArray.from_array(x)
+        out = []
+        for plan in (p, q):
+            dy = spb.DeviceArray.from_array(np.zeros(m.nrows, dt))
+            plan.spmv_dev(dx.ptr, dy.ptr)
+            out.append(dy.to_array(dt, m.nrows))
+            dy.free()
+        dx.free()
+        assert np.array_equal(np.isnan(out[0]), np.isnan(out[1]))
+        assert np.array_equal(np.isinf(out[0]), np.isinf(out[1]))
+        assert np.array_equal(np.sign(out[0][np.isinf(out[0])]), np.sign(out[1][np.isinf(out[1])]))
+        if not bad:
+            want = out[0] if want is None else want
+            assert np.array_equal(out[0], want)
+    p.free()
+    q.free()
+
+
+@pytest.mark.parametrize("kind", ["L", "D", "S"])
+def test_reference_entries_run_windowed_tiles(kind):
+    """Build_VNEC_L / D / S on scattered columns run windowed tiles; y matches
+    the oracle's rows."""
+    m = g.rmat(13, 16, seed=14)
+    A = spb.Matrix.from_csr(m.nrows, m.ncols, m.ptr, m.col, m.val)
+    plan = spb.build_vnec(kind, A)
+    lib = spb.L.load()
+    assert lib.vnec_plan_windowed(spb.C.c_void_p(lib.VNEC_plan_of_ext(spb.C.cast(plan, spb.C.c_void_p))))
+    y = spb.Vector(m.nrows)
+    assert spb.spmv_vnec(kind, y, A, spb.Vector.from_array(m.x), plan) == ""
+    ok, worst = _check(m, y.to_array(), "fp64")
+    assert ok, worst
+    spb.free_vnec(kind, plan)
+
+
+def test_window_relabelled_columns_beyond_the_training_sizes():
+    """Above 2^24 nonzeros and 2 MiB of x the learned mode may relabel the
+    columns of windowed tiles hot-first: the same sums either way."""
+    m = g.uniform(2_100_011, 8, seed=15)
+    A = spb.Matrix.from_csr(m.nrows, m.ncols, m.ptr, m.col, m.val)
+    assert m.nnz > 1 << 24
+    p = spb.Plan(A, "learned")
+    assert _windowed(p)
+    dx = spb.DeviceArray.from_array(m.x)
+    dy = spb.DeviceArray(8 * m.nrows)
+    p.spmv_dev(dx.ptr, dy.ptr)
+    ok, worst = _check(m, dy.to_array(np.float64, m.nrows), "fp64")
+    assert ok, (p.info(), worst)
+    p.free()

@@ -187,6 +187,7 @@ static void matrix_drop_device(spb_csr *a)
     a->feat_ready = 0;
     a->pattern_ready = 0;
     a->refined_slice_ipt = 0;
+    a->window_relabel = 0;
 }
 
 SpB_Info SpB_Matrix_free(SpB_Matrix *A)

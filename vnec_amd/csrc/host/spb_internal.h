@@ -61,6 +61,8 @@ typedef struct spb_csr {
     int refined_slice_ipt; /* slice-family pick measured at this ipt (0: not
                               yet): the fastest of S at it and variant G  */
     int refined_slice_variant, refined_slice_ipt_out;
+    int window_relabel; /* windowed tiles faster over relabelled columns:
+                           1 no, 2 yes (0: not measured)                */
     int feat_ready;     /* feat_ints holds the selector's statistics     */
     int pattern_ready;  /* pattern_rows holds the count below            */
     int64_t pattern_rows; /* rows that fit the dominant column-offset pattern */
@@ -148,6 +150,17 @@ struct vnec_plan_s {
     int32_t *cperm;     /* ncols */
     int32_t *rcol;      /* nnz   */
     double *xperm;      /* ncols */
+    /* windowed tiles (vnec_hip_spmv_win) run in place of the kernel tune
+       names when w_threads > 0 (vnec_win_args describes the arrays) */
+    int w_threads, w_ipt; /* threads per tile, items per thread          */
+    int w_entries;        /* LDS entries of the largest tile             */
+    int64_t w_window;     /* window entries over all tiles               */
+    double *w_val;
+    float *w_hi, *w_lo;
+    uint16_t *w_rank, *w_rbase, *w_off;
+    uint32_t *w_flags;
+    uint64_t *w_rmask;
+    int32_t *w_win, *w_base, *w_desc;
     /* borrowed from the matrix mirror */
     const int32_t *ptr, *col;
     const double *val;
@@ -204,6 +217,26 @@ SpB_Info vnec_pattern_coverage(spb_csr *a, int64_t *nregular);
 SpB_Info vnec_plan_run(struct vnec_plan_s *p, const void *x_dev, void *y_dev);
 double vnec_slice_padding(const spb_csr *a);
 
+/* As vnec_plan_build_ext, for a plan shape the library chose itself: it may
+ * run as windowed tiles. */
+SpB_Info vnec_plan_build_chosen(vnec_plan *plan, const SpB_Matrix A, const vnec_tuning *t);
+
+/* ---- windowed tiles (spb_window.c) ---- */
+/* Whether a chosen plan t of a runs as windowed tiles. */
+int vnec_window_applies(const spb_csr *a, const vnec_tuning *t);
+/* Adds VNEC_LANES_RELABEL to the L or C plan t when windowed tiles of a are
+ * faster over hot-first relabelled columns (measured, cached on a; only
+ * where x is large and a has more than 2^24 nonzeros). */
+SpB_Info vnec_window_relabel(spb_csr *a, vnec_tuning *t);
+/* Builds p's windowed tiles (p->col: the columns, relabelled or not). */
+SpB_Info vnec_window_build(struct vnec_plan_s *p, const spb_csr *a);
+SpB_Info vnec_window_launch(const struct vnec_plan_s *p, const void *x_dev, void *y_dev, hipStream_t s);
+/* Bytes of the arrays the kernel reads per launch (x and y aside). */
+int64_t vnec_window_bytes(const struct vnec_plan_s *p);
+void vnec_window_release(struct vnec_plan_s *p);
+/* Whether the plan runs as windowed tiles. */
+int vnec_plan_windowed(vnec_plan plan);
+
 /* ---- autotuner and selector (spb_tune.c) ---- */
 /* Tuning chosen by a selection mode (vnec_select_mode) for FP64 values
  * and nrhs right-hand sides (several: the merge-path kernel, its
@@ -241,6 +274,8 @@ SpB_Info vnec_refine_slice_plan(spb_csr *a, vnec_tuning *t);
  * merged column runs a workgroup's 256 rows read, staged in LDS when they
  * total at most VNEC_PATTERN_WIN_MAX entries (else wsize = 0). */
 void vnec_pattern_window(const int32_t *pat, int L, vnec_pattern_args *g);
+/* Best of three hipGraph-timed means of `iters` SpMVs of plan p. */
+SpB_Info vnec_time_plan(vnec_plan p, const void *dx, void *dy, int iters, double *ms_out);
 int vnec_csort_rule(spb_csr *a);
 
 /* ---- compiled-in selector model (spb_selector_model.c, generated) ---- */

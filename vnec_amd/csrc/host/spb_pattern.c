@@ -272,7 +272,7 @@ SpB_Info vnec_pattern_build(struct vnec_plan_s *p, spb_csr *a)
             }
             t.encoding = enc;
         }
-        if (rc == SpB_SUCCESS) rc = vnec_plan_build_ext(&p->g_subplan, p->g_sub, &t);
+        if (rc == SpB_SUCCESS) rc = vnec_plan_build_chosen(&p->g_subplan, p->g_sub, &t);
         if (rc == SpB_SUCCESS) {
             p->g_ysub = (double *)vnec_malloc_dev(sizeof(double) * (size_t)nirr, &p->dev_bytes);
             if (!p->g_ysub) rc = SpB_FAILURE;

@@ -87,6 +87,7 @@ static void plan_release(struct vnec_plan_s *p)
     vnec_free_dev(p->hcol);
     vnec_free_dev(p->hot_order);
     vnec_free_dev(p->xhot);
+    vnec_window_release(p);
     memset(p, 0, sizeof *p);
 }
 
@@ -449,7 +450,10 @@ int vnec_pattern_rule(spb_csr *a)
     return (double)nreg >= 0.9 * (double)a->base.row && (double)a->nnz >= 0.8 * slots;
 }
 
-SpB_Info vnec_plan_build_ext(vnec_plan *plan, const SpB_Matrix A, const vnec_tuning *t)
+/* t's plan; with windowed != 0 it may run as windowed tiles where they
+ * apply (spb_window.c): the modes that choose a plan ask for that, a caller
+ * that names a plan shape gets that shape. */
+static SpB_Info plan_build(vnec_plan *plan, const SpB_Matrix A, const vnec_tuning *t, int windowed)
 {
     if (!plan) return vnec_fail("vnec_plan_build_ext: NULL plan handle");
     *plan = NULL;
@@ -503,7 +507,10 @@ SpB_Info vnec_plan_build_ext(vnec_plan *plan, const SpB_Matrix A, const vnec_tun
             tune.lanes = 64;
         }
         const int mode = t ? t->variant : VNEC_SELECT_LEARNED;
-        if ((tune.variant == VNEC_VAR_L || tune.variant == VNEC_VAR_C) && tune.nrhs == 1 &&
+        if (mode != VNEC_SELECT_LEARNED && mode != VNEC_SELECT_AUTOTUNE) windowed = 0;
+        if (windowed && vnec_window_applies(a, &tune)) {
+            if (vnec_window_relabel(a, &tune) != SpB_SUCCESS) return SpB_FAILURE;
+        } else if ((tune.variant == VNEC_VAR_L || tune.variant == VNEC_VAR_C) && tune.nrhs == 1 &&
             tune.encoding == VNEC_ENC_FP64) {
             /* CSR-ordered or column-sorted tiles, persistent or with
              * per-tile carries, at the chosen granularity: the rule mode
@@ -598,6 +605,7 @@ SpB_Info vnec_plan_build_ext(vnec_plan *plan, const SpB_Matrix A, const vnec_tun
                              tune.ipt, tune.encoding, tune.nrhs);
     }
     if (spb_matrix_upload(a) != SpB_SUCCESS) return SpB_FAILURE;
+    windowed = windowed && vnec_window_applies(a, &tune);
 
     struct vnec_plan_s *p = (struct vnec_plan_s *)calloc(1, sizeof *p);
     if (!p) return vnec_fail("out of memory");
@@ -615,7 +623,11 @@ SpB_Info vnec_plan_build_ext(vnec_plan *plan, const SpB_Matrix A, const vnec_tun
     p->ntiles = M > 0 ? (M + T - 1) / T : 0;
     hipStream_t s = vnec_stream();
     SpB_Info rc = SpB_SUCCESS;
-    if (tune.variant == VNEC_VAR_S) {
+    if (windowed) {
+        p->tune.grid = -1;
+        if (plan_relabelled(&p->tune)) rc = build_relabel(p, a);
+        if (rc == SpB_SUCCESS) rc = vnec_window_build(p, a);
+    } else if (tune.variant == VNEC_VAR_S) {
         p->ntiles = 0;
         p->tune.grid = -1;
         rc = p->nrows > 0 ? build_slices(p, a) : SpB_SUCCESS;
@@ -710,6 +722,16 @@ SpB_Info vnec_plan_build_ext(vnec_plan *plan, const SpB_Matrix A, const vnec_tun
     return SpB_SUCCESS;
 }
 
+SpB_Info vnec_plan_build_ext(vnec_plan *plan, const SpB_Matrix A, const vnec_tuning *t)
+{
+    return plan_build(plan, A, t, !t || t->variant < 0);
+}
+
+SpB_Info vnec_plan_build_chosen(vnec_plan *plan, const SpB_Matrix A, const vnec_tuning *t)
+{
+    return plan_build(plan, A, t, 1);
+}
+
 /* Bytes of one value slot in the plan's encoding. */
 static int64_t value_bytes(int enc) { return enc == VNEC_ENC_HI || enc == VNEC_ENC_FP32 ? 4 : 8; }
 
@@ -724,6 +746,7 @@ static int64_t main_kernel_bytes(const struct vnec_plan_s *p)
     const int64_t nr = p->nrows, nc = p->ncols, nnz = p->nnz;
     const int64_t vecs = xb * k * (nc + nr), coords = 8 * (p->ntiles + 1);
     const int64_t windows = 8 * p->nruns + 4 * (p->ntiles + 1) + 4 * p->ntiles; /* runs, run_off, nec */
+    if (p->w_threads > 0) return vnec_window_bytes(p) + vecs;
     switch (p->tune.variant) {
     case VNEC_VAR_G:
         return p->g_nslices * 64 * (int64_t)p->g_L * vb + 4 * nr + vecs;
@@ -937,6 +960,7 @@ static SpB_Info launch_d(struct vnec_plan_s *p, const void *x_dev, void *y_dev, 
 static SpB_Info launch_main(struct vnec_plan_s *p, const vnec_merge_args *m, const void *x_dev,
                             void *y_dev, hipStream_t s)
 {
+    if (p->w_threads > 0) return vnec_window_launch(p, x_dev, y_dev, s);
     if (p->tune.variant == VNEC_VAR_G) {
         vnec_pattern_args g;
         g.masks = p->g_masks;
@@ -980,6 +1004,7 @@ static SpB_Info launch_main(struct vnec_plan_s *p, const vnec_merge_args *m, con
 static SpB_Info launch_fixup(struct vnec_plan_s *p, const void *x_dev, void *y_dev, hipStream_t s)
 {
     if (p->tune.variant == VNEC_VAR_S) return SpB_SUCCESS; /* row-aligned tiles: no carries */
+    if (p->w_threads > 0) return SpB_SUCCESS;                   /* cut rows meet in the kernel */
     if (p->tune.variant == VNEC_VAR_G) { /* the irregular rows */
         if (!p->g_nirr) return SpB_SUCCESS;
         if (vnec_plan_run(p->g_subplan, x_dev, p->g_ysub) != SpB_SUCCESS) return SpB_FAILURE;

@@ -659,6 +659,18 @@ static SpB_Info autotune_multi(spb_csr *a, int nrhs, int *ipt)
     return rc;
 }
 
+SpB_Info vnec_time_plan(vnec_plan p, const void *dx, void *dy, int iters, double *ms_out)
+{
+    SpB_Info rc = SpB_SUCCESS;
+    *ms_out = INFINITY;
+    for (int r = 0; rc == SpB_SUCCESS && r < 3; r++) {
+        double ms = 0.0;
+        rc = vnec_time_dev_ext(p, dx, dy, iters, 1, 0, &ms);
+        if (rc == SpB_SUCCESS && ms < *ms_out) *ms_out = ms;
+    }
+    return rc;
+}
+
 /* Best of three hipGraph-timed means of `iters` SpMVs of plan tuning u on
  * a (INFINITY when u does not build). */
 static SpB_Info time_tuning(spb_csr *a, const vnec_tuning *u, const void *dx, void *dy, int iters,
@@ -670,12 +682,7 @@ static SpB_Info time_tuning(spb_csr *a, const vnec_tuning *u, const void *dx, vo
         vnec_clear_error(); /* not a contender */
         return SpB_SUCCESS;
     }
-    SpB_Info rc = SpB_SUCCESS;
-    for (int r = 0; rc == SpB_SUCCESS && r < 3; r++) {
-        double ms = 0.0;
-        rc = vnec_time_dev_ext(p, dx, dy, iters, 1, 0, &ms);
-        if (rc == SpB_SUCCESS && ms < *ms_out) *ms_out = ms;
-    }
+    SpB_Info rc = vnec_time_plan(p, dx, dy, iters, ms_out);
     vnec_plan_free_ext(&p);
     return rc;
 }

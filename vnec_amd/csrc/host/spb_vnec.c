@@ -449,7 +449,7 @@ static struct vnec_plan_s *gpu_plan_for(spb_csr *a, plan_kind kind)
         /* FP64 otherwise: the learned selector, whose candidates include
          * the D blocks at widths 4, 8 and 16 */
     }
-    if (vnec_plan_build_ext(&p, (SpB_Matrix)a, &t) != SpB_SUCCESS) return NULL;
+    if (vnec_plan_build_chosen(&p, (SpB_Matrix)a, &t) != SpB_SUCCESS) return NULL;
     return p;
 }
 

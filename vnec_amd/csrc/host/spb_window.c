@@ -1,0 +1,279 @@
+/*
+ * spb_window.c — plans of windowed tiles (vnec_win.hip): where they run, how
+ * large their tiles are, and their layout.
+ *
+ * A selection mode's pick (spb_tune.c) names a plan shape; where windowed
+ * tiles apply they run in place of the kernel it names, over the same matrix
+ * with the same arithmetic, and the plan keeps reporting the pick.
+ */
+#include <math.h>
+#include <stdlib.h>
+#include <string.h>
+
+#include "spb_internal.h"
+
+/* Runs of consecutive columns: the window's gathers are contiguous loads. */
+static int contiguous(const spb_csr *a)
+{
+    uint64_t v[VNEC_NFEAT_INTS];
+    if (vnec_feature_ints_ext((SpB_Matrix)a, v) == SpB_SUCCESS) return v[VF_NEC_LARGE] >= 8 * v[VF_RUNS_LARGE];
+    vnec_clear_error();
+    return 0;
+}
+
+/* Over such columns FP64 64-row slices stream better than windowed tiles from
+ * this many nonzeros on (banded and block-diagonal matrices of 16.8M nonzeros:
+ * slices 29.9-32.4 us, windowed 31.0-33.1; of 8.9M 19.1 against 17.9, of 13.7M
+ * 27.6 against 26.7).  FP32 slices never do (16.8M: 21.7-83 against 19.0-23). */
+#define WINDOW_SLICE_NNZ ((int64_t)15 << 20)
+
+int vnec_window_applies(const spb_csr *a, const vnec_tuning *t)
+{
+    if (a->nnz == 0 || t->nrhs > 1) return 0;
+    switch (t->variant) {
+    case VNEC_VAR_L:
+    case VNEC_VAR_C:
+    case VNEC_VAR_E:
+    case VNEC_VAR_D:
+        return 1;
+    case VNEC_VAR_S:
+        return t->encoding == VNEC_ENC_FP32 || (int64_t)a->nnz < WINDOW_SLICE_NNZ || !contiguous(a);
+    default: /* pattern slices read no columns at all */
+        return 0;
+    }
+}
+
+/* Nonzeros per thread.  Few nonzeros: small tiles, so that there are enough
+ * workgroups (R-MAT 14, 0.08M: 4.3 us at 4, 4.7 at 8, 5.9 at 16; 0.39M
+ * uniform 4.8 / 5.4 / 6.9; 0.55M R-MAT 6.1 / 5.8 / 6.7; 1.4M R-MAT 9.1 / 9.1 /
+ * 8.0; 3.9M 22.7 / 20.4 / 18.4).  Two or three nonzeros a row: as many row
+ * sums as window entries in LDS (1.3M over 0.7M rows 16.3 / 18.4 / 17.4).
+ * Runs of consecutive columns in FP64: the gathers are cheap and the smaller
+ * tiles overlap better (16.8M banded 44.6 / 31.0 / 33.8; FP32 35.5 / 21.9 /
+ * 19.0). */
+static int window_ipt(const spb_csr *a, int enc)
+{
+    const int64_t nnz = (int64_t)a->nnz, nr = (int64_t)a->base.row;
+    if (nnz < 450000 || nnz < 3 * nr) return 4;
+    if (nnz < 1100000) return 8;
+    if (enc != VNEC_ENC_FP32 && contiguous(a)) return 8;
+    return 16;
+}
+
+/* LDS of a workgroup up to which two fit a compute unit. */
+#define WINDOW_LDS_TWO (80 * 1024 - 256)
+
+static void window_args(const struct vnec_plan_s *p, const void *x_dev, void *y_dev, vnec_win_args *w)
+{
+    memset(w, 0, sizeof *w);
+    w->desc = p->w_desc;
+    w->ntiles = p->ntiles;
+    w->entries = p->w_entries;
+    w->win = p->w_win;
+    w->wbase = p->w_base;
+    w->woff = p->w_off;
+    w->wv = p->w_val;
+    w->whi = p->w_hi;
+    w->wlo = p->w_lo;
+    w->wl = p->w_rank;
+    w->wt = p->w_flags;
+    w->rmask = p->w_rmask;
+    w->rbase = p->w_rbase;
+    if (p->tune.encoding == VNEC_ENC_FP32) {
+        w->x32 = (const float *)x_dev;
+        w->y32 = (float *)y_dev;
+        w->slot32 = (float *)p->carry; /* ntiles doubles hold ntiles floats */
+    } else {
+        w->x = (const double *)x_dev;
+        w->y = (double *)y_dev;
+        w->slot = p->carry;
+    }
+    w->ipt = p->w_ipt;
+    w->encoding = p->tune.encoding;
+}
+
+void vnec_window_release(struct vnec_plan_s *p)
+{
+    void **own[] = {(void **)&p->w_val,   (void **)&p->w_hi,    (void **)&p->w_lo,   (void **)&p->w_rank,
+                    (void **)&p->w_rbase, (void **)&p->w_flags, (void **)&p->w_rmask, (void **)&p->w_win,
+                    (void **)&p->w_base,  (void **)&p->w_desc,  (void **)&p->w_off};
+    for (size_t i = 0; i < sizeof own / sizeof own[0]; i++) {
+        vnec_free_dev(*own[i]);
+        *own[i] = NULL;
+    }
+}
+
+/* A tile boundary fewer than this many nonzeros into a row moves to the row's
+ * start, and the tiles are that much shorter than T: fewer cut rows (a slot
+ * that stays empty is not read).  T / 16, or T / 64 where that saves a round
+ * of resident workgroups (R-MAT 18, 518 tiles of 7680 against 493 of 8064 on
+ * 512 workgroups: 20.3 against 17.8 us; power-law rows 59.0 against 52.9). */
+static int window_snap(int64_t T, int64_t weight, int enc)
+{
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
+        cus = 256;
+    const int64_t wgs = (int64_t)cus * (T > 4096 && enc != VNEC_ENC_FP32 ? 2 : 4);
+    const int64_t s16 = T - T / 16, s64 = T - T / 64;
+    const int64_t p16 = (weight + s16 - 1) / s16, p64 = (weight + s64 - 1) / s64;
+    return (int)((p64 + wgs - 1) / wgs < (p16 + wgs - 1) / wgs ? T / 64 : T / 16);
+}
+
+static SpB_Info build_at(struct vnec_plan_s *p, const spb_csr *a, int ipt)
+{
+    hipStream_t s = vnec_stream();
+    const int64_t T = VNEC_WIN_THREADS * (int64_t)ipt, nnz = p->nnz;
+    const int enc = p->tune.encoding;
+    const int snap = window_snap(T, nnz + p->nrows / VNEC_WIN_ROWS, enc);
+    const int64_t step = T - snap, P = (nnz + p->nrows / VNEC_WIN_ROWS + step - 1) / step;
+    const size_t slots = (size_t)(P * T), esz = enc == VNEC_ENC_FP32 ? sizeof(float) : sizeof(double);
+    const size_t words = (size_t)(p->nrows / 64 + P + 1), chunks = (size_t)(nnz / 64 + P + 1);
+    int64_t bytes = 0;
+    p->ntiles = P;
+    p->w_threads = VNEC_WIN_THREADS;
+    p->w_ipt = ipt;
+    p->coords = (int32_t *)vnec_malloc_dev(sizeof(int32_t) * 2 * (size_t)(P + 1), &bytes);
+    p->carry = (double *)vnec_malloc_dev(sizeof(double) * (size_t)P, &bytes);
+    p->w_desc = (int32_t *)vnec_malloc_dev(sizeof(int32_t) * 8 * (size_t)P, &bytes);
+    p->w_win = (int32_t *)vnec_malloc_dev(sizeof(int32_t) * (size_t)nnz, NULL);
+    p->w_base = (int32_t *)vnec_malloc_dev(sizeof(int32_t) * chunks, NULL);
+    p->w_off = (uint16_t *)vnec_malloc_dev(sizeof(uint16_t) * 64 * chunks, NULL);
+    if (enc == VNEC_ENC_FP64) p->w_val = (double *)vnec_malloc_dev(sizeof(double) * slots, &bytes);
+    else p->w_hi = (float *)vnec_malloc_dev(sizeof(float) * slots, &bytes);
+    if (enc == VNEC_ENC_HILO) p->w_lo = (float *)vnec_malloc_dev(sizeof(float) * slots, &bytes);
+    p->w_rank = (uint16_t *)vnec_malloc_dev(sizeof(uint16_t) * slots, &bytes);
+    p->w_flags = (uint32_t *)vnec_malloc_dev(sizeof(uint32_t) * (size_t)(P * VNEC_WIN_THREADS), &bytes);
+    p->w_rmask = (uint64_t *)vnec_malloc_dev(sizeof(uint64_t) * words, &bytes);
+    p->w_rbase = (uint16_t *)vnec_malloc_dev(sizeof(uint16_t) * words, &bytes);
+    int32_t *tmp = (int32_t *)vnec_malloc_dev(sizeof(int32_t) * (size_t)(2 * P + 2), NULL);
+    uint16_t *lcol = (uint16_t *)vnec_malloc_dev(sizeof(uint16_t) * (size_t)nnz, NULL);
+    int32_t *nec = tmp, *nsum = tmp + P, *mx_dev = tmp + 2 * P;
+    int32_t mx[2] = {0, 0}; /* LDS entries; whether a distance passes 16 bits */
+    int32_t *hnec = (int32_t *)malloc(sizeof(int32_t) * (size_t)P);
+    SpB_Info rc = p->coords && p->carry && p->w_desc && p->w_win && p->w_base && p->w_off &&
+                          (enc == VNEC_ENC_FP64 ? (void *)p->w_val : (void *)p->w_hi) &&
+                          (enc != VNEC_ENC_HILO || p->w_lo) && p->w_rank && p->w_flags && p->w_rmask &&
+                          p->w_rbase && tmp && lcol
+                      ? SpB_SUCCESS : SpB_FAILURE;
+    if (rc == SpB_SUCCESS && !hnec) rc = vnec_fail("out of memory");
+    if (rc == SpB_SUCCESS)
+        rc = vnec_hip_ok(vnec_hip_win_coords(a->d_ptr, p->nrows, nnz, P, step, snap, p->coords, s), "window tiles");
+    if (rc == SpB_SUCCESS) /* (nsum: scratch for the run counts) */
+        rc = vnec_hip_ok(vnec_hip_ecr_tiles_pass1(p->col, p->coords, P, lcol, NULL, p->w_win, nec, nsum, s),
+                         "windows");
+    if (rc == SpB_SUCCESS)
+        rc = vnec_hip_ok(vnec_hip_win_desc(a->d_ptr, p->nrows, p->coords, P, nec, p->w_desc, s), "window rows");
+    if (rc == SpB_SUCCESS) rc = vnec_hip_ok(hipMemsetAsync(mx_dev, 0, sizeof mx, s), "memset");
+    if (rc == SpB_SUCCESS)
+        rc = vnec_hip_ok(vnec_hip_win_list(p->coords, P, p->w_win, nec, p->w_base, p->w_off, mx_dev + 1, s),
+                         "window lists");
+    if (rc == SpB_SUCCESS)
+        rc = vnec_hip_ok(vnec_hip_win_layout(a->d_ptr, a->d_val, lcol, p->coords, P, ipt, enc, p->w_val, p->w_hi,
+                                             p->w_lo, p->w_rank, p->w_flags, p->w_rmask, p->w_rbase, nec, nsum,
+                                             mx_dev, p->carry, s), "window layout");
+    if (rc == SpB_SUCCESS)
+        rc = vnec_hip_ok(hipMemcpyAsync(mx, mx_dev, sizeof mx, hipMemcpyDeviceToHost, s), "d2h");
+    if (rc == SpB_SUCCESS)
+        rc = vnec_hip_ok(hipMemcpyAsync(hnec, nec, sizeof(int32_t) * (size_t)P, hipMemcpyDeviceToHost, s), "d2h");
+    if (rc == SpB_SUCCESS) rc = vnec_hip_ok(hipStreamSynchronize(s), "window sync");
+    vnec_free_dev(tmp);
+    vnec_free_dev(lcol);
+    if (rc == SpB_SUCCESS) {
+        p->w_window = 0;
+        for (int64_t t = 0; t < P; t++) p->w_window += hnec[t];
+        p->w_entries = mx[0];
+        if (mx[1]) {
+            vnec_free_dev(p->w_base);
+            vnec_free_dev(p->w_off);
+            p->w_base = NULL;
+            p->w_off = NULL;
+            bytes += (int64_t)sizeof(int32_t) * nnz;
+        } else {
+            vnec_free_dev(p->w_win);
+            p->w_win = NULL;
+            bytes += (int64_t)((sizeof(int32_t) + 64 * sizeof(uint16_t)) * chunks);
+        }
+        if (ipt > 8 && (size_t)(p->w_entries + 1) * esz > WINDOW_LDS_TWO) {
+            /* half the tile, so that two workgroups fit a compute unit */
+            vnec_window_release(p);
+            vnec_free_dev(p->coords);
+            vnec_free_dev(p->carry);
+            p->coords = NULL;
+            p->carry = NULL;
+            free(hnec);
+            return build_at(p, a, 8);
+        }
+        vnec_win_args w;
+        window_args(p, NULL, NULL, &w);
+        rc = vnec_hip_ok(vnec_hip_win_prepare(&w), "window LDS");
+    }
+    p->dev_bytes += bytes;
+    free(hnec);
+    return rc;
+}
+
+SpB_Info vnec_window_build(struct vnec_plan_s *p, const spb_csr *a)
+{
+    return build_at(p, a, window_ipt(a, p->tune.encoding));
+}
+
+SpB_Info vnec_window_launch(const struct vnec_plan_s *p, const void *x_dev, void *y_dev, hipStream_t s)
+{
+    vnec_win_args w;
+    window_args(p, x_dev, y_dev, &w);
+    return vnec_hip_ok(vnec_hip_spmv_win(&w, s), "window kernel");
+}
+
+int64_t vnec_window_bytes(const struct vnec_plan_s *p)
+{
+    const int enc = p->tune.encoding;
+    const int64_t vb = enc == VNEC_ENC_HI || enc == VNEC_ENC_FP32 ? 4 : 8, P = p->ntiles;
+    /* values and ranks, the window's columns, the threads' flags, the row
+     * masks and the tile descriptors */
+    return p->nnz * (vb + 2) + p->w_window * (p->w_off ? 2 : 4) + (p->w_off ? p->w_window / 16 : 0) +
+           4 * (p->nnz + p->w_ipt - 1) / p->w_ipt + 10 * (p->nrows / 64 + P) + 32 * P;
+}
+
+int vnec_plan_windowed(vnec_plan plan) { return plan && plan->magic == SPB_MAGIC_PLAN && plan->w_threads > 0; }
+
+/* Relabelled columns are measured from this size of x and this many nonzeros
+ * on (R-MAT 22 with dense rows, x 32 MiB: 494.9 us plain, 388.7 relabelled
+ * with the permutation of x; R-MAT 20, x 8 MiB: 78.4 either way; below, the
+ * permutation costs more than the lines it saves: R-MAT 18 17.8 -> 20.7). */
+#define WINDOW_RELABEL_X ((int64_t)1 << 21)
+#define WINDOW_RELABEL_NNZ ((int64_t)1 << 24)
+
+SpB_Info vnec_window_relabel(spb_csr *a, vnec_tuning *t)
+{
+    const int64_t nr = (int64_t)a->base.row, nc = (int64_t)a->base.col;
+    if ((t->variant != VNEC_VAR_L && t->variant != VNEC_VAR_C) || t->encoding != VNEC_ENC_FP64 ||
+        8 * nc < WINDOW_RELABEL_X || (int64_t)a->nnz <= WINDOW_RELABEL_NNZ)
+        return SpB_SUCCESS;
+    const int lanes = (t->lanes == 64 ? 0 : t->lanes) | VNEC_LANES_RELABEL;
+    if (!a->window_relabel) {
+        double *dx = (double *)vnec_malloc_dev(sizeof(double) * (size_t)nc, NULL);
+        double *dy = (double *)vnec_malloc_dev(sizeof(double) * (size_t)nr, NULL);
+        SpB_Info rc = dx && dy ? SpB_SUCCESS : SpB_FAILURE;
+        if (rc == SpB_SUCCESS) rc = vnec_hip_ok(vnec_hip_zero_f64(dx, nc, vnec_stream()), "zero x");
+        double ms[2] = {INFINITY, INFINITY};
+        for (int k = 0; rc == SpB_SUCCESS && k < 2; k++) {
+            vnec_tuning u = *t;
+            if (k) u.lanes = lanes;
+            vnec_plan p = NULL;
+            if (vnec_plan_build_chosen(&p, (SpB_Matrix)a, &u) != SpB_SUCCESS) {
+                if (!k) rc = SpB_FAILURE;
+                else vnec_clear_error(); /* not a contender */
+                continue;
+            }
+            rc = vnec_time_plan(p, dx, dy, 20, &ms[k]);
+            vnec_plan_free_ext(&p);
+        }
+        vnec_free_dev(dx);
+        vnec_free_dev(dy);
+        if (rc != SpB_SUCCESS) return rc;
+        a->window_relabel = ms[1] < ms[0] ? 2 : 1;
+    }
+    if (a->window_relabel == 2) t->lanes = lanes;
+    return SpB_SUCCESS;
+}
