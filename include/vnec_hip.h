@@ -213,7 +213,7 @@ int vnec_hip_merge_supported(int variant, int ipt, int encoding, int nrhs);
  * thread k holding nonzeros k ipt .. k ipt + ipt - 1 of the tile. */
 #define VNEC_WIN_THREADS 512
 #define VNEC_WIN_MAX_IPT 16 /* ipt: 4, 8 or 16                              */
-#define VNEC_WIN_ROWS 8     /* rows that weigh as much as a nonzero         */
+#define VNEC_WIN_ROW8 1     /* eight rows weigh as much as a nonzero        */
 typedef struct {
     const int32_t *desc;    /* 8 per tile: first row, first nonzero, rows
                                ended, nonzeros, distinct columns, and of the
@@ -246,8 +246,9 @@ typedef struct {
     int ipt, encoding;
 } vnec_win_args;
 /* Tile boundaries (coords, 2 (P + 1) ints) every `step` units of nonzeros
- * plus rows / VNEC_WIN_ROWS; step + snap <= VNEC_WIN_THREADS * ipt. */
-int vnec_hip_win_coords(const int32_t *ptr, int64_t nrows, int64_t nnz, int64_t P, int64_t step, int snap,
+ * plus rows row8 / 8 (row8: VNEC_WIN_ROW8 for windowed tiles); a tile holds
+ * fewer than step + snap nonzeros.  vnec_hip_win_desc: nec may be NULL. */
+int vnec_hip_win_coords(const int32_t *ptr, int64_t nrows, int64_t nnz, int64_t P, int row8, int64_t step, int snap,
                         int32_t *coords, void *stream);
 int vnec_hip_win_desc(const int32_t *ptr, int64_t nrows, const int32_t *coords, int64_t ntiles, const int32_t *nec,
                       int32_t *desc, void *stream);
@@ -264,6 +265,37 @@ int vnec_hip_win_layout(const int32_t *ptr, const double *val, const uint16_t *l
 /* Lets the kernel of these arguments use the LDS it needs (once per plan). */
 int vnec_hip_win_prepare(const vnec_win_args *a);
 int vnec_hip_spmv_win(const vnec_win_args *a, void *stream);
+
+/* Several right-hand sides (k = 2, 4, 8 or 16, FP64 values) over tiles of
+ * streams of `run` nonzeros walked by Q = min(4, k / 2) lanes (vnec_spmm.hip):
+ * a tile has NS = 256 / Q streams and T = NS run slots. */
+#define VNEC_SPMM_MAX_ITEMS 4096
+#define VNEC_SPMM_MAX_ROWS 4096 /* rows of a tile: T 8 / row8 + 8 at most    */
+typedef struct {
+    const int32_t *desc;   /* 8 per tile, as vnec_win_args                  */
+    int64_t ntiles;
+    const double *sv;      /* T per tile, [load][stream][lane][2]: nonzero
+                              stream run + 2 Q load + 2 lane + e            */
+    const int32_t *sc;     /* T per tile, [load][stream][lane][4]: columns  */
+    const uint32_t *sf;    /* 2 per stream: row-end flags, the ordinal of
+                              its first row end in the tile                 */
+    const uint64_t *rmask; /* as vnec_win_args                              */
+    const int32_t *rbase;
+    const int32_t *nsum;   /* row sums of each tile, an unfinished last row
+                              included                                      */
+    int sums;              /* most row sums of a tile                       */
+    const double *x;       /* [ncols][k], 16-byte aligned                   */
+    double *y;             /* [nrows][k], 16-byte aligned, or with ldy > 0  */
+    int64_t ldy;           /* k columns of nrows, ldy apart                 */
+    double *slot;          /* [ntiles][k] partial sums of cut rows          */
+    int64_t ncols;
+    int k, run;
+} vnec_spmm_args;
+int vnec_hip_spmm_layout(const int32_t *ptr, const int32_t *col, const double *val, const int32_t *coords,
+                         int64_t ntiles, int k, int run, double *sv, int32_t *sc, uint32_t *sf, uint64_t *rmask,
+                         int32_t *rbase, int32_t *nsum, int32_t *max_dev, double *slot, void *stream);
+int vnec_hip_spmm_prepare(const vnec_spmm_args *a);
+int vnec_hip_spmm_tiles(const vnec_spmm_args *a, void *stream);
 
 /* Gather-ceiling probe over a matrix's values and columns (nnz): with
  * gather = 0 it streams them, with gather = 1 it also gathers x[col] per

@@ -200,12 +200,15 @@ SIGNATURES = {
     "vnec_hip_carry_fixup": (C.c_int, [vp, vp, i64, vp, i64, C.c_int, vp]),
     "vnec_hip_carry_fixup_f32": (C.c_int, [vp, vp, i64, vp, i64, vp]),
     "vnec_hip_merge_supported": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int]),
-    "vnec_hip_win_coords": (C.c_int, [vp, i64, i64, i64, i64, C.c_int, vp, vp]),
+    "vnec_hip_win_coords": (C.c_int, [vp, i64, i64, i64, C.c_int, i64, C.c_int, vp, vp]),
     "vnec_hip_win_desc": (C.c_int, [vp, i64, vp, i64, vp, vp, vp]),
     "vnec_hip_win_list": (C.c_int, [vp, i64, vp, vp, vp, vp, vp, vp]),
     "vnec_hip_win_layout": (C.c_int, [vp, vp, vp, vp, i64, C.c_int, C.c_int] + [vp] * 12),
     "vnec_hip_win_prepare": (C.c_int, [vp]),
     "vnec_hip_spmv_win": (C.c_int, [vp, vp]),
+    "vnec_hip_spmm_layout": (C.c_int, [vp, vp, vp, vp, i64, C.c_int, C.c_int] + [vp] * 9),
+    "vnec_hip_spmm_prepare": (C.c_int, [vp]),
+    "vnec_hip_spmm_tiles": (C.c_int, [vp, vp]),
     "vnec_hip_stream_grid": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int)]),
     "vnec_hip_stream_supported": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int]),
     "vnec_hip_spmv_stream": (C.c_int, [vp, C.c_int, vp, vp, vp]),

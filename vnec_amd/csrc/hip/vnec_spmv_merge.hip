@@ -230,66 +230,6 @@ __device__ __forceinline__ void store_rhs(double *p, const double (&v)[2])
     *(double2 *)p = make_double2(v[0], v[1]);
 }
 
-// Segmented scan over merge-path streams of Q lanes each (lane q of a
-// stream holds columns [q VW, q VW + VW) of the stream's (flag, tail)):
-// Hillis-Steele steps of Q, 2Q, ... lanes within the wavefront, then the
-// wavefronts chained in order through LDS.  cin = carry into the stream's
-// head row, incl = the stream's inclusive value (the last stream's closes
-// the tile).  s_v: VNEC_NWAVES * Q * VW doubles, s_f: VNEC_NWAVES ints.
-template <int Q, int VW>
-__device__ __forceinline__ void stream_seg_carry(int flag, const double (&tail)[VW], int *s_f, double *s_v,
-                                                 double (&cin)[VW], double (&incl)[VW])
-{
-    constexpr int K = Q * VW;
-    const int lane = lane_id(), w = wave_id(), q = lane % Q;
-    int f = flag;
-    double v[VW];
-#pragma unroll
-    for (int e = 0; e < VW; e++) v[e] = tail[e];
-#pragma unroll
-    for (int off = Q; off < VNEC_WAVE; off <<= 1) {
-        const int fu = __shfl_up(f, off, VNEC_WAVE);
-        double vu[VW];
-#pragma unroll
-        for (int e = 0; e < VW; e++) vu[e] = __shfl_up(v[e], off, VNEC_WAVE);
-        if (lane >= off) {
-            if (!f) {
-#pragma unroll
-                for (int e = 0; e < VW; e++) v[e] = vu[e] + v[e];
-            }
-            f |= fu;
-        }
-    }
-    if (lane >= VNEC_WAVE - Q) {
-#pragma unroll
-        for (int e = 0; e < VW; e++) s_v[w * K + q * VW + e] = v[e];
-        if (q == 0) s_f[w] = f;
-    }
-    __syncthreads();
-    if (threadIdx.x < Q) {
-        double c[VW];
-#pragma unroll
-        for (int e = 0; e < VW; e++) c[e] = 0.0;
-        for (int k = 0; k < VNEC_NWAVES; k++) {
-            const int fw = s_f[k];
-#pragma unroll
-            for (int e = 0; e < VW; e++) {
-                const double tw = s_v[k * K + q * VW + e];
-                s_v[k * K + q * VW + e] = c[e];  // carry into wavefront k
-                c[e] = fw ? tw : c[e] + tw;
-            }
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int e = 0; e < VW; e++) {
-        const double cw = s_v[w * K + q * VW + e];
-        incl[e] = f ? v[e] : v[e] + cw;
-        const double prev = __shfl_up(incl[e], Q, VNEC_WAVE);
-        cin[e] = lane < Q ? cw : prev;
-    }
-}
-
 // Multi-RHS (variant L), grouped lanes: x is [ncols][K], y is [nrows][K].
 // Values, columns and row ends are staged in LDS as in k_spmv_mergeK; the
 // tile's merge items are then cut into VNEC_BLOCK / Q streams of Q IPT

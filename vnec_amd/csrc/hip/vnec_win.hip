@@ -16,7 +16,7 @@
 // The walk is then a multiply-add and a bit test per nonzero out of registers
 // and LDS: no row pointers, no search, no staged products.  Row sums go to y
 // through LDS, 64 consecutive rows per store, empty rows included.  A row cut
-// by a tile boundary is joined in the kernel (win_meet), so the SpMV is one
+// by a tile boundary is joined in the kernel (vnec_meet.h), so the SpMV is one
 // launch.
 //
 // Measured on one MI355X, kernel and carry fix-up of the column-sorted plans
@@ -36,19 +36,20 @@
 
 #include "vnec_common.h"
 #include "vnec_hip.h"
+#include "vnec_meet.h"
 
 #define WIN_NT VNEC_WIN_THREADS
 #define WIN_NW (WIN_NT / VNEC_WAVE)
 
 // ------------------------------------------------------------- builders
-// Tile boundaries: rows and nonzeros merged with VNEC_WIN_ROWS rows weighing
-// as much as one nonzero, cut every `step` units, so a tile holds at most
-// `step` nonzeros and VNEC_WIN_ROWS (step + 1) rows.  W(r) = ptr[r] +
-// r / VNEC_WIN_ROWS is the weight before row r; the boundary at weight d lies
-// in the last row with W <= d.  With snap > 0 a boundary fewer than snap
-// nonzeros into a row moves to the row's start.
+// Tile boundaries: rows and nonzeros merged, eight rows weighing as much as
+// row8 nonzeros, cut every `step` units, so a tile holds at most `step`
+// nonzeros and 8 (step + 1) / row8 rows.  W(r) = ptr[r] + r row8 / 8 is the
+// weight before row r; the boundary at weight d lies in the last row with
+// W <= d.  With snap > 0 a boundary fewer than snap nonzeros into a row moves
+// to the row's start.
 __global__ void k_win_coords(const int32_t *__restrict__ ptr, int64_t nrows, int64_t nnz, int64_t P,
-                             int64_t step, int snap, int2 *__restrict__ co)
+                             int row8, int64_t step, int snap, int2 *__restrict__ co)
 {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t > P) return;
@@ -60,14 +61,17 @@ __global__ void k_win_coords(const int32_t *__restrict__ ptr, int64_t nrows, int
     int64_t lo = 0, hi = nrows;  // last row with W(row) <= d
     while (lo < hi) {
         const int64_t mid = (lo + hi + 1) >> 1;
-        if (ptr[mid] + mid / VNEC_WIN_ROWS <= d) lo = mid; else hi = mid - 1;
+        if (ptr[mid] + mid * row8 / 8 <= d) lo = mid; else hi = mid - 1;
     }
-    int64_t y = d - lo / VNEC_WIN_ROWS;
+    int64_t y = d - lo * row8 / 8;
     if (lo == nrows) {
         y = nnz;
     } else {
         if (y - ptr[lo] < snap) y = ptr[lo];
-        if (y >= ptr[lo + 1]) lo++;  // the row is complete
+        if (y >= ptr[lo + 1]) {  // the row is complete
+            y = ptr[lo + 1];
+            lo++;
+        }
     }
     co[t] = make_int2((int)lo, (int)y);
 }
@@ -85,7 +89,7 @@ __device__ __forceinline__ int64_t win_tile_of(const int2 *co, int64_t P, int64_
     return lo;
 }
 
-__global__ void k_win_meet(const int32_t *__restrict__ ptr, int64_t nrows, const int2 *__restrict__ co, int64_t P,
+__global__ void k_win_desc(const int32_t *__restrict__ ptr, int64_t nrows, const int2 *__restrict__ co, int64_t P,
                            int4 *__restrict__ desc, const int32_t *__restrict__ nec)
 {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -100,7 +104,7 @@ __global__ void k_win_meet(const int32_t *__restrict__ ptr, int64_t nrows, const
     if (c1.x < nrows && ptr[c1.x] < c1.y && (c1.x != c0.x || !m.y))
         m.z = (int)(win_tile_of(co, P, ptr[c1.x + 1] - 1) - t + 1);
     desc[2 * t] = make_int4(c0.x, c0.y, c1.x - c0.x, c1.y - c0.y);
-    desc[2 * t + 1] = make_int4(nec[t], m.x, m.y, m.z);
+    desc[2 * t + 1] = make_int4(nec ? nec[t] : 0, m.x, m.y, m.z);
 }
 
 // Window lists in 16 bits: per 64 entries the first column (wbase) and each
@@ -219,22 +223,12 @@ __global__ void k_win_max(const int32_t *__restrict__ a, int64_t n, int32_t *__r
     if (lane_id() == 0) atomicMax(out, m);
 }
 
-// Slots of the partial sums of cut rows, empty.
-#define WIN_EMPTY64 0x7FF4DEADBEEF0001ull  // a NaN no sum is stored as
-#define WIN_EMPTY32 0x7FA4DEADu
-__global__ void k_win_empty(int64_t n, int fp32, void *__restrict__ slot)
-{
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    if (fp32) ((uint32_t *)slot)[i] = WIN_EMPTY32;
-    else ((uint64_t *)slot)[i] = WIN_EMPTY64;
-}
-
-extern "C" int vnec_hip_win_coords(const int32_t *ptr, int64_t nrows, int64_t nnz, int64_t P, int64_t step,
-                                   int snap, int32_t *coords, void *stream)
+extern "C" int vnec_hip_win_coords(const int32_t *ptr, int64_t nrows, int64_t nnz, int64_t P, int row8,
+                                   int64_t step, int snap, int32_t *coords, void *stream)
 {
     const unsigned g = (unsigned)((P + 256) / 256);
-    hipLaunchKernelGGL(k_win_coords, dim3(g), dim3(256), 0, (hipStream_t)stream, ptr, nrows, nnz, P, step, snap,
+    hipLaunchKernelGGL(k_win_coords, dim3(g), dim3(256), 0, (hipStream_t)stream, ptr, nrows, nnz, P, row8, step,
+                       snap,
                        (int2 *)coords);
     return (int)hipGetLastError();
 }
@@ -242,7 +236,7 @@ extern "C" int vnec_hip_win_coords(const int32_t *ptr, int64_t nrows, int64_t nn
 extern "C" int vnec_hip_win_desc(const int32_t *ptr, int64_t nrows, const int32_t *coords, int64_t ntiles,
                                  const int32_t *nec, int32_t *desc, void *stream)
 {
-    hipLaunchKernelGGL(k_win_meet, dim3((unsigned)((ntiles + 255) / 256)), dim3(256), 0, (hipStream_t)stream, ptr,
+    hipLaunchKernelGGL(k_win_desc, dim3((unsigned)((ntiles + 255) / 256)), dim3(256), 0, (hipStream_t)stream, ptr,
                        nrows, (const int2 *)coords, ntiles, (int4 *)desc, nec);
     return (int)hipGetLastError();
 }
@@ -268,7 +262,7 @@ extern "C" int vnec_hip_win_layout(const int32_t *ptr, const double *val, const 
     int64_t g = (ntiles + 255) / 256;
     if (g > 256) g = 256;
     hipLaunchKernelGGL(k_win_max, dim3((unsigned)g), dim3(256), 0, s, (const int32_t *)nsum, ntiles, max_dev);
-    hipLaunchKernelGGL(k_win_empty, dim3((unsigned)((ntiles + 255) / 256)), dim3(256), 0, s, ntiles, esz == 4, slot);
+    hipLaunchKernelGGL(k_meet_empty, dim3((unsigned)((ntiles + 255) / 256)), dim3(256), 0, s, ntiles, esz == 4, slot);
     return (int)hipGetLastError();
 }
 
@@ -353,50 +347,6 @@ __device__ __forceinline__ double read_lane(double v, int l)
 __device__ __forceinline__ float read_lane(float v, int l)
 {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
-}
-
-// Partial sums of a row cut by tile boundaries meet pairwise: the row's n
-// tiles are the leaves of a binary tree whose node between leaves m - 1 and m
-// owns slot[t0 + m].  Of a node's two sides the first to arrive leaves its sum
-// in the slot and is done; the second takes it, empties the slot for the next
-// launch and goes on with the total.  The tree fixes the order of the sums,
-// one atomic exchange carries both the value and its arrival, and nothing is
-// waited for.
-__device__ __forceinline__ bool win_swap(double *slot, double &s)
-{
-    typedef unsigned long long u64;
-    const u64 mine = s != s ? 0x7FF8000000000000ull : (u64)__double_as_longlong(s);
-    const u64 old = __hip_atomic_exchange((u64 *)slot, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (old == WIN_EMPTY64) return false;
-    __hip_atomic_store((u64 *)slot, WIN_EMPTY64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    s += __longlong_as_double((long long)old);
-    return true;
-}
-__device__ __forceinline__ bool win_swap(float *slot, float &s)
-{
-    const uint32_t mine = s != s ? 0x7FC00000u : (uint32_t)__float_as_int(s);
-    const uint32_t old = __hip_atomic_exchange((uint32_t *)slot, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (old == WIN_EMPTY32) return false;
-    __hip_atomic_store((uint32_t *)slot, WIN_EMPTY32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    s += __int_as_float((int)old);
-    return true;
-}
-
-template <typename F>
-__device__ __forceinline__ void win_meet(F *slot, int t0, int n, int leaf, F s, F *yrow)
-{
-    int i = leaf;  // first leaf of the node whose sum is s
-    for (int z = 1; z < n; z <<= 1) {
-        int m = i + z;  // first leaf of the node's right side
-        if (i & z) {
-            m = i;
-            i -= z;
-        } else if (m >= n) {
-            continue;  // no right side
-        }
-        if (!win_swap(slot + t0 + m, s)) return;
-    }
-    *yrow = s;
 }
 
 template <int IPT, int ENC, bool W16>
@@ -537,12 +487,12 @@ __global__ __launch_bounds__(WIN_NT) void k_spmv_win(vnec_win_args a, int grid)
     if (flags) s_y[ord0] += cin;
     F *slot = win_slot(a, F());
     if (tid == WIN_NT - 1) {  // the tile's last, partial row
-        if (d1.w) win_meet(slot, t, d1.w, 0, blk, y + x0 + nrow);
-        else if (d1.z && nrow == 0) win_meet(slot, d1.y, d1.z, t - d1.y, blk, y + x0);
+        if (d1.w) meet_rows(slot, 1, t, d1.w, 0, blk, y + x0 + nrow);
+        else if (d1.z && nrow == 0) meet_rows(slot, 1, d1.y, d1.z, t - d1.y, blk, y + x0);
     }
     __syncthreads();
     if (tid == 0 && d1.z && nrow > 0)  // its first row, begun in an earlier tile
-        win_meet(slot, d1.y, d1.z, t - d1.y, s_y[0], y + x0);
+        meet_rows(slot, 1, d1.y, d1.z, t - d1.y, s_y[0], y + x0);
 
     // the tile's rows, 64 at a time
     for (int q0 = w; q0 * VNEC_WAVE < nrow; q0 += NW * VNEC_WAVE) {

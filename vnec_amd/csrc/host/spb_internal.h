@@ -161,6 +161,15 @@ struct vnec_plan_s {
     uint32_t *w_flags;
     uint64_t *w_rmask;
     int32_t *w_win, *w_base, *w_desc;
+    /* several right-hand sides: stream tiles (vnec_hip_spmm_tiles) in place of
+       the merge-path kernel when m_run > 0 and x and y are 16-byte aligned
+       (vnec_spmm_args describes the arrays) */
+    int m_run, m_sums;
+    int64_t m_ntiles;
+    double *m_val, *m_slot;
+    int32_t *m_col, *m_desc, *m_rbase, *m_nsum;
+    uint32_t *m_flags;
+    uint64_t *m_rmask;
     /* borrowed from the matrix mirror */
     const int32_t *ptr, *col;
     const double *val;
@@ -234,7 +243,15 @@ SpB_Info vnec_window_launch(const struct vnec_plan_s *p, const void *x_dev, void
 /* Bytes of the arrays the kernel reads per launch (x and y aside). */
 int64_t vnec_window_bytes(const struct vnec_plan_s *p);
 void vnec_window_release(struct vnec_plan_s *p);
-/* Whether the plan runs as windowed tiles. */
+/* Stream tiles of a chosen plan with several right-hand sides. */
+int vnec_streams_apply(const spb_csr *a, const vnec_tuning *t);
+SpB_Info vnec_streams_build(struct vnec_plan_s *p, const spb_csr *a);
+/* Whether p's launch on these vectors takes them. */
+int vnec_streams_run(const struct vnec_plan_s *p, const void *x_dev, const void *y_dev);
+/* ldy: 0, or the distance of y's columns when they lie one after another. */
+SpB_Info vnec_streams_launch(const struct vnec_plan_s *p, const void *x_dev, void *y_dev, int64_t ldy, hipStream_t s);
+int64_t vnec_streams_bytes(const struct vnec_plan_s *p);
+/* Whether the plan runs as windowed or stream tiles. */
 int vnec_plan_windowed(vnec_plan plan);
 
 /* ---- autotuner and selector (spb_tune.c) ---- */

@@ -493,7 +493,10 @@ static SpB_Info plan_build(vnec_plan *plan, const SpB_Matrix A, const vnec_tunin
         tune = g;
     } else {
         int nrhs = t && t->nrhs > 0 ? t->nrhs : 1;
-        if (vnec_select_tuning(a, t ? t->variant : VNEC_SELECT_LEARNED, nrhs, &tune) != SpB_SUCCESS)
+        int smode = t ? t->variant : VNEC_SELECT_LEARNED;
+        /* (stream tiles leave the merge-path kernel's granularity unused) */
+        if (nrhs > 1 && windowed && (!t || t->encoding == VNEC_ENC_FP64)) smode = VNEC_SELECT_LEARNED;
+        if (vnec_select_tuning(a, smode, nrhs, &tune) != SpB_SUCCESS)
             return SpB_FAILURE;
         if (t) tune.encoding = t->encoding;
         /* a candidate without a kernel for the requested encoding falls back
@@ -605,6 +608,7 @@ static SpB_Info plan_build(vnec_plan *plan, const SpB_Matrix A, const vnec_tunin
                              tune.ipt, tune.encoding, tune.nrhs);
     }
     if (spb_matrix_upload(a) != SpB_SUCCESS) return SpB_FAILURE;
+    const int streams = windowed && vnec_streams_apply(a, &tune);
     windowed = windowed && vnec_window_applies(a, &tune);
 
     struct vnec_plan_s *p = (struct vnec_plan_s *)calloc(1, sizeof *p);
@@ -676,6 +680,7 @@ static SpB_Info plan_build(vnec_plan *plan, const SpB_Matrix A, const vnec_tunin
         if (rc == SpB_SUCCESS)
             rc = vnec_hip_ok(vnec_hip_partition(a->d_ptr, p->nrows, p->nnz, p->ntiles, 0, p->coords, s),
                              "partition");
+        if (rc == SpB_SUCCESS && streams) rc = vnec_streams_build(p, a);
         if (rc == SpB_SUCCESS && plan_relabelled(&p->tune)) rc = build_relabel(p, a);
         if (rc == SpB_SUCCESS && tune.variant == VNEC_VAR_D) rc = build_d(p, a);
         if (rc == SpB_SUCCESS && tune.variant == VNEC_VAR_H) rc = build_hot(p, a);
@@ -729,7 +734,9 @@ SpB_Info vnec_plan_build_ext(vnec_plan *plan, const SpB_Matrix A, const vnec_tun
 
 SpB_Info vnec_plan_build_chosen(vnec_plan *plan, const SpB_Matrix A, const vnec_tuning *t)
 {
-    return plan_build(plan, A, t, 1);
+    if (plan_build(plan, A, t, 1) == SpB_SUCCESS) return SpB_SUCCESS;
+    vnec_clear_error();
+    return plan_build(plan, A, t, 0);
 }
 
 /* Bytes of one value slot in the plan's encoding. */
@@ -747,6 +754,7 @@ static int64_t main_kernel_bytes(const struct vnec_plan_s *p)
     const int64_t vecs = xb * k * (nc + nr), coords = 8 * (p->ntiles + 1);
     const int64_t windows = 8 * p->nruns + 4 * (p->ntiles + 1) + 4 * p->ntiles; /* runs, run_off, nec */
     if (p->w_threads > 0) return vnec_window_bytes(p) + vecs;
+    if (p->m_run > 0) return vnec_streams_bytes(p) + vecs;
     switch (p->tune.variant) {
     case VNEC_VAR_G:
         return p->g_nslices * 64 * (int64_t)p->g_L * vb + 4 * nr + vecs;
@@ -961,6 +969,7 @@ static SpB_Info launch_main(struct vnec_plan_s *p, const vnec_merge_args *m, con
                             void *y_dev, hipStream_t s)
 {
     if (p->w_threads > 0) return vnec_window_launch(p, x_dev, y_dev, s);
+    if (vnec_streams_run(p, x_dev, y_dev)) return vnec_streams_launch(p, x_dev, y_dev, 0, s);
     if (p->tune.variant == VNEC_VAR_G) {
         vnec_pattern_args g;
         g.masks = p->g_masks;
@@ -1004,7 +1013,8 @@ static SpB_Info launch_main(struct vnec_plan_s *p, const vnec_merge_args *m, con
 static SpB_Info launch_fixup(struct vnec_plan_s *p, const void *x_dev, void *y_dev, hipStream_t s)
 {
     if (p->tune.variant == VNEC_VAR_S) return SpB_SUCCESS; /* row-aligned tiles: no carries */
-    if (p->w_threads > 0) return SpB_SUCCESS;                   /* cut rows meet in the kernel */
+    if (p->w_threads > 0 || vnec_streams_run(p, x_dev, y_dev))
+        return SpB_SUCCESS; /* cut rows meet in the kernel */
     if (p->tune.variant == VNEC_VAR_G) { /* the irregular rows */
         if (!p->g_nirr) return SpB_SUCCESS;
         if (vnec_plan_run(p->g_subplan, x_dev, p->g_ysub) != SpB_SUCCESS) return SpB_FAILURE;
@@ -1101,16 +1111,21 @@ SpB_Info vnec_spmm_colmajor_dev_ext(vnec_plan plan, const void *X_dev, void *Y_d
     if (!plan || plan->magic != SPB_MAGIC_PLAN) return vnec_fail("vnec_spmm_colmajor_dev_ext: not a plan");
     const int k = plan->tune.nrhs;
     if (k <= 1) return vnec_plan_run(plan, X_dev, Y_dev);
+    const int streams = plan->m_run > 0; /* these write Y's columns themselves */
     if (!plan->xt) {
         plan->xt = (double *)vnec_malloc_dev(sizeof(double) * (size_t)(plan->ncols > 0 ? plan->ncols * k : 1),
                                              &plan->dev_bytes);
+        if (!plan->xt) return SpB_FAILURE;
+    }
+    if (!streams && !plan->yt) {
         plan->yt = (double *)vnec_malloc_dev(sizeof(double) * (size_t)(plan->nrows > 0 ? plan->nrows * k : 1),
                                              &plan->dev_bytes);
-        if (!plan->xt || !plan->yt) return SpB_FAILURE;
+        if (!plan->yt) return SpB_FAILURE;
     }
     hipStream_t s = vnec_stream();
     if (vnec_hip_ok(vnec_hip_rhs_layout((const double *)X_dev, plan->ncols, k, 1, plan->xt, s), "interleave X"))
         return SpB_FAILURE;
+    if (streams) return vnec_streams_launch(plan, plan->xt, Y_dev, plan->nrows, s);
     if (vnec_plan_run(plan, plan->xt, plan->yt) != SpB_SUCCESS) return SpB_FAILURE;
     return vnec_hip_ok(vnec_hip_rhs_layout(plan->yt, plan->nrows, k, 0, (double *)Y_dev, s), "de-interleave Y");
 }

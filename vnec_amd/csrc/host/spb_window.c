@@ -1,6 +1,7 @@
 /*
- * spb_window.c — plans of windowed tiles (vnec_win.hip): where they run, how
- * large their tiles are, and their layout.
+ * spb_window.c — plans of windowed tiles (vnec_win.hip) and, for several
+ * right-hand sides, of stream tiles (vnec_spmm.hip): where they run, how large
+ * their tiles are, and their layout.
  *
  * A selection mode's pick (spb_tune.c) names a plan shape; where windowed
  * tiles apply they run in place of the kernel it names, over the same matrix
@@ -96,7 +97,9 @@ void vnec_window_release(struct vnec_plan_s *p)
 {
     void **own[] = {(void **)&p->w_val,   (void **)&p->w_hi,    (void **)&p->w_lo,   (void **)&p->w_rank,
                     (void **)&p->w_rbase, (void **)&p->w_flags, (void **)&p->w_rmask, (void **)&p->w_win,
-                    (void **)&p->w_base,  (void **)&p->w_desc,  (void **)&p->w_off};
+                    (void **)&p->w_base,  (void **)&p->w_desc,  (void **)&p->w_off,   (void **)&p->m_val,
+                    (void **)&p->m_slot,  (void **)&p->m_col,   (void **)&p->m_desc,  (void **)&p->m_rbase,
+                    (void **)&p->m_nsum,  (void **)&p->m_flags, (void **)&p->m_rmask};
     for (size_t i = 0; i < sizeof own / sizeof own[0]; i++) {
         vnec_free_dev(*own[i]);
         *own[i] = NULL;
@@ -125,8 +128,8 @@ static SpB_Info build_at(struct vnec_plan_s *p, const spb_csr *a, int ipt)
     hipStream_t s = vnec_stream();
     const int64_t T = VNEC_WIN_THREADS * (int64_t)ipt, nnz = p->nnz;
     const int enc = p->tune.encoding;
-    const int snap = window_snap(T, nnz + p->nrows / VNEC_WIN_ROWS, enc);
-    const int64_t step = T - snap, P = (nnz + p->nrows / VNEC_WIN_ROWS + step - 1) / step;
+    const int snap = window_snap(T, nnz + p->nrows * VNEC_WIN_ROW8 / 8, enc);
+    const int64_t step = T - snap, P = (nnz + p->nrows * VNEC_WIN_ROW8 / 8 + step - 1) / step;
     const size_t slots = (size_t)(P * T), esz = enc == VNEC_ENC_FP32 ? sizeof(float) : sizeof(double);
     const size_t words = (size_t)(p->nrows / 64 + P + 1), chunks = (size_t)(nnz / 64 + P + 1);
     int64_t bytes = 0;
@@ -158,7 +161,7 @@ static SpB_Info build_at(struct vnec_plan_s *p, const spb_csr *a, int ipt)
                       ? SpB_SUCCESS : SpB_FAILURE;
     if (rc == SpB_SUCCESS && !hnec) rc = vnec_fail("out of memory");
     if (rc == SpB_SUCCESS)
-        rc = vnec_hip_ok(vnec_hip_win_coords(a->d_ptr, p->nrows, nnz, P, step, snap, p->coords, s), "window tiles");
+        rc = vnec_hip_ok(vnec_hip_win_coords(a->d_ptr, p->nrows, nnz, P, VNEC_WIN_ROW8, step, snap, p->coords, s), "window tiles");
     if (rc == SpB_SUCCESS) /* (nsum: scratch for the run counts) */
         rc = vnec_hip_ok(vnec_hip_ecr_tiles_pass1(p->col, p->coords, P, lcol, NULL, p->w_win, nec, nsum, s),
                          "windows");
@@ -235,7 +238,11 @@ int64_t vnec_window_bytes(const struct vnec_plan_s *p)
            4 * (p->nnz + p->w_ipt - 1) / p->w_ipt + 10 * (p->nrows / 64 + P) + 32 * P;
 }
 
-int vnec_plan_windowed(vnec_plan plan) { return plan && plan->magic == SPB_MAGIC_PLAN && plan->w_threads > 0; }
+int vnec_plan_windowed(vnec_plan plan)
+{
+    return plan && plan->magic == SPB_MAGIC_PLAN && (plan->w_threads > 0 || plan->m_run > 0);
+}
+
 
 /* Relabelled columns are measured from this size of x and this many nonzeros
  * on (R-MAT 22 with dense rows, x 32 MiB: 494.9 us plain, 388.7 relabelled
@@ -276,4 +283,106 @@ SpB_Info vnec_window_relabel(spb_csr *a, vnec_tuning *t)
     }
     if (a->window_relabel == 2) t->lanes = lanes;
     return SpB_SUCCESS;
+}
+
+/* ------------------------------------------------ several right-hand sides */
+/* With 4 and 8 right-hand sides and this many nonzeros (and weighted rows) a
+ * stream is 32 nonzeros long instead of 16 (batch of 28.7M: k = 4 178 us at 16,
+ * 170 at 32; k = 8 188, 179; uniform 4.2M: 49.1, 50.2 and 66.2, 66.8; R-MAT 18
+ * 35.0, 33.7 and 38.1, 38.5; R-MAT 17, 1.9M: 16.9, 18.2 and 20.7, 20.1).  k = 2
+ * takes 8 and k = 16 takes 16 throughout: the batch 157 at 8, 163 at 16 for k =
+ * 2; uniform 80.9 at 16, 80.4 at 32 for k = 16. */
+#define STREAMS_LONG_RUNS ((int64_t)1 << 23)
+
+int vnec_streams_apply(const spb_csr *a, const vnec_tuning *t)
+{
+    return a->nnz > 0 && t->variant == VNEC_VAR_L && t->encoding == VNEC_ENC_FP64 &&
+           (t->nrhs == 2 || t->nrhs == 4 || t->nrhs == 8 || t->nrhs == 16);
+}
+
+/* Eight rows weigh as much as this many nonzeros: a tile's row sums, k to a
+ * row, stay within 32 KiB of LDS. */
+static int streams_row8(int k) { return k == 16 ? 64 : 32; }
+
+SpB_Info vnec_streams_build(struct vnec_plan_s *p, const spb_csr *a)
+{
+    hipStream_t s = vnec_stream();
+    const int k = p->tune.nrhs, q = k < 8 ? k / 2 : 4, row8 = streams_row8(k);
+    const int64_t nnz = p->nnz, weight = nnz + p->nrows * row8 / 8;
+    const int run = k == 2 ? 8 : k < 16 && weight >= STREAMS_LONG_RUNS ? 32 : 16;
+    const int64_t T = (int64_t)256 / q * run;
+    const int snap = (int)(T / 32);
+    const int64_t P = (weight + T - snap - 1) / (T - snap), step = (weight + P - 1) / P, words = p->nrows / 64 + P + 1;
+    int64_t *acct = &p->dev_bytes;
+    p->m_val = (double *)vnec_malloc_dev(sizeof(double) * (size_t)(P * T), acct);
+    p->m_col = (int32_t *)vnec_malloc_dev(sizeof(int32_t) * (size_t)(P * T), acct);
+    p->m_flags = (uint32_t *)vnec_malloc_dev(sizeof(uint32_t) * 2 * (size_t)(P * (256 / q)), acct);
+    p->m_rmask = (uint64_t *)vnec_malloc_dev(sizeof(uint64_t) * (size_t)words, acct);
+    p->m_rbase = (int32_t *)vnec_malloc_dev(sizeof(int32_t) * (size_t)words, acct);
+    p->m_desc = (int32_t *)vnec_malloc_dev(sizeof(int32_t) * 8 * (size_t)P, acct);
+    p->m_nsum = (int32_t *)vnec_malloc_dev(sizeof(int32_t) * (size_t)(P + 1), acct);
+    p->m_slot = (double *)vnec_malloc_dev(sizeof(double) * (size_t)(P * k), acct);
+    int32_t *co = (int32_t *)vnec_malloc_dev(sizeof(int32_t) * 2 * (size_t)(P + 1), NULL);
+    int32_t mx = 0, *mx_dev = p->m_nsum ? p->m_nsum + P : NULL;
+    SpB_Info rc = p->m_val && p->m_col && p->m_flags && p->m_rmask && p->m_rbase && p->m_desc && p->m_nsum &&
+                          p->m_slot && co
+                      ? SpB_SUCCESS : SpB_FAILURE;
+    if (rc == SpB_SUCCESS)
+        rc = vnec_hip_ok(vnec_hip_win_coords(a->d_ptr, p->nrows, nnz, P, row8, step, snap, co, s), "stream tiles");
+    if (rc == SpB_SUCCESS)
+        rc = vnec_hip_ok(vnec_hip_win_desc(a->d_ptr, p->nrows, co, P, NULL, p->m_desc, s), "stream rows");
+    if (rc == SpB_SUCCESS) rc = vnec_hip_ok(hipMemsetAsync(mx_dev, 0, sizeof mx, s), "memset");
+    if (rc == SpB_SUCCESS)
+        rc = vnec_hip_ok(vnec_hip_spmm_layout(a->d_ptr, a->d_col, a->d_val, co, P, k, run, p->m_val, p->m_col,
+                                              p->m_flags, p->m_rmask, p->m_rbase, p->m_nsum, mx_dev, p->m_slot, s),
+                         "stream layout");
+    if (rc == SpB_SUCCESS) rc = vnec_hip_ok(hipMemcpyAsync(&mx, mx_dev, sizeof mx, hipMemcpyDeviceToHost, s), "d2h");
+    if (rc == SpB_SUCCESS) rc = vnec_hip_ok(hipStreamSynchronize(s), "stream sync");
+    vnec_free_dev(co);
+    if (rc == SpB_SUCCESS) {
+        vnec_spmm_args m;
+        memset(&m, 0, sizeof m);
+        m.k = k;
+        m.run = run;
+        m.sums = mx;
+        rc = vnec_hip_ok(vnec_hip_spmm_prepare(&m), "stream LDS");
+    }
+    p->m_ntiles = P;
+    p->m_run = run;
+    p->m_sums = mx;
+    return rc;
+}
+
+int vnec_streams_run(const struct vnec_plan_s *p, const void *x_dev, const void *y_dev)
+{
+    return p->m_run > 0 && !(((uintptr_t)x_dev | (uintptr_t)y_dev) & 15);
+}
+
+SpB_Info vnec_streams_launch(const struct vnec_plan_s *p, const void *x_dev, void *y_dev, int64_t ldy, hipStream_t s)
+{
+    vnec_spmm_args m;
+    memset(&m, 0, sizeof m);
+    m.desc = p->m_desc;
+    m.ntiles = p->m_ntiles;
+    m.sv = p->m_val;
+    m.sc = p->m_col;
+    m.sf = p->m_flags;
+    m.rmask = p->m_rmask;
+    m.rbase = p->m_rbase;
+    m.nsum = p->m_nsum;
+    m.sums = p->m_sums;
+    m.x = (const double *)x_dev;
+    m.y = (double *)y_dev;
+    m.ldy = ldy;
+    m.slot = p->m_slot;
+    m.ncols = p->ncols;
+    m.k = p->tune.nrhs;
+    m.run = p->m_run;
+    return vnec_hip_ok(vnec_hip_spmm_tiles(&m, s), "stream kernel");
+}
+
+int64_t vnec_streams_bytes(const struct vnec_plan_s *p)
+{
+    return 12 * p->nnz + 8 * (p->nnz + p->m_run - 1) / p->m_run + 12 * (p->nrows / 64 + p->m_ntiles) +
+           36 * p->m_ntiles;
 }
