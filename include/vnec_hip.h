@@ -213,6 +213,7 @@ int vnec_hip_merge_supported(int variant, int ipt, int encoding, int nrhs);
  * thread k holding nonzeros k ipt .. k ipt + ipt - 1 of the tile. */
 #define VNEC_WIN_THREADS 512
 #define VNEC_WIN_MAX_IPT 16 /* ipt: 4, 8 or 16                              */
+#define VNEC_WIN_WIDE (1 << 30) /* of a distinct-column count               */
 #define VNEC_WIN_ROW8 1     /* eight rows weigh as much as a nonzero        */
 typedef struct {
     const int32_t *desc;    /* 8 per tile: first row, first nonzero, rows
@@ -223,8 +224,9 @@ typedef struct {
     int64_t ntiles;
     int entries;            /* LDS entries of the largest tile              */
     const int32_t *win;     /* distinct columns, tile t's ascending from its
-                               first nonzero's index on; or, when woff is
-                               given, 16 bits each:                         */
+                               first nonzero's index on; when woff is given
+                               (x below 4 GiB), read only for tiles whose
+                               count carries VNEC_WIN_WIDE; the others':    */
     const int32_t *wbase;   /* the first of every 64 and                    */
     const uint16_t *woff;   /* each one's distance from it, tile t's from
                                chunk (first nonzero >> 6) + t on            */
@@ -252,9 +254,10 @@ int vnec_hip_win_coords(const int32_t *ptr, int64_t nrows, int64_t nnz, int64_t 
                         int32_t *coords, void *stream);
 int vnec_hip_win_desc(const int32_t *ptr, int64_t nrows, const int32_t *coords, int64_t ntiles, const int32_t *nec,
                       int32_t *desc, void *stream);
-/* wbase / woff from the windows uniq / nec of vnec_hip_ecr_tiles_pass1;
- * *wide (caller-zeroed) is set when a distance does not fit 16 bits. */
-int vnec_hip_win_list(const int32_t *coords, int64_t ntiles, const int32_t *uniq, const int32_t *nec, int32_t *wbase,
+/* wbase / woff from the windows uniq / nec of vnec_hip_ecr_tiles_pass1; sets
+ * VNEC_WIN_WIDE in nec where a distance does not fit 16 bits, and then *wide
+ * (caller-zeroed). */
+int vnec_hip_win_list(const int32_t *coords, int64_t ntiles, const int32_t *uniq, int32_t *nec, int32_t *wbase,
                       uint16_t *woff, int32_t *wide, void *stream);
 /* Slots, flags, masks, per-tile LDS entries (nsum) and their maximum
  * (*max_dev, caller-zeroed); empties the slots of partial sums. */

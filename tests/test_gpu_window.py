@@ -72,10 +72,18 @@ def _lds_limit():  # rows of one nonzero, then rows of six
     return _rows(lens, 1 << 20, 13, cols=rng.integers(0, 1 << 20, int(lens.sum())))
 
 
+def _mixed_wide():  # long rows of consecutive columns beside rows over eight million columns
+    rng = np.random.default_rng(14)
+    lens = [3] * 900 + [9000] + [3] * 900 + [70] * 60 + [2] * 40
+    cols = [np.sort(rng.integers(0, 8_000_000 if n == 3 else 20_000, n)) if n < 9000 else np.arange(n) for n in lens]
+    return _rows(lens, 8_000_000, 14, cols=np.concatenate(cols))
+
+
 MATRICES = {
     "one": lambda: _rows([1], 1, 1),
     "edge2047": lambda: _tile_edge(2047), "edge2048": lambda: _tile_edge(2048), "edge2049": lambda: _tile_edge(2049),
     "cut_rows": _cut_rows, "empty_stretches": _empty_stretches, "sparse_window": _sparse_window,
+    "mixed_wide": _mixed_wide,
     "repeated_descending": _repeated_descending,
     "ipt8": lambda: g.powerlaw(60013, 2.2, 3, 20000, seed=9),   # 4096-item tiles, long rows
     "ipt16": lambda: g.rmat(17, 12, seed=10),                   # 8192-item tiles

@@ -108,10 +108,11 @@ __global__ void k_win_desc(const int32_t *__restrict__ ptr, int64_t nrows, const
 }
 
 // Window lists in 16 bits: per 64 entries the first column (wbase) and each
-// entry's distance from it.  *wide is set when a distance does not fit.
+// entry's distance from it.  A tile with a distance that does not fit (a long
+// row's dense piece beside a few scattered columns) is read from uniq instead:
+// nec[t] gets VNEC_WIN_WIDE, and *wide is set.
 __global__ __launch_bounds__(VNEC_BLOCK) void k_win_list(const int2 *__restrict__ co, int64_t ntiles,
-                                                         const int32_t *__restrict__ uniq,
-                                                         const int32_t *__restrict__ nec,
+                                                         const int32_t *__restrict__ uniq, int32_t *__restrict__ nec,
                                                          int32_t *__restrict__ wbase, uint16_t *__restrict__ woff,
                                                          int32_t *__restrict__ wide)
 {
@@ -126,7 +127,10 @@ __global__ __launch_bounds__(VNEC_BLOCK) void k_win_list(const int2 *__restrict_
         woff[c0 * 64 + i] = (uint16_t)(c - b);
         bad |= c - b > 65535;
     }
-    if (bad) atomicOr(wide, 1);
+    if (__syncthreads_or(bad) && threadIdx.x == 0) {
+        nec[t] = n | VNEC_WIN_WIDE;
+        atomicOr(wide, 1);
+    }
 }
 
 // Values, window ranks, row-end flags and row masks of the tiles, in the
@@ -171,7 +175,7 @@ __global__ __launch_bounds__(VNEC_BLOCK) void k_win_layout(
         }
         run += tot;
     }
-    if (tid == 0) nsum[t] = nec[t] + 1 + run;  // entries of LDS
+    if (tid == 0) nsum[t] = (nec[t] & ~VNEC_WIN_WIDE) + 1 + run;  // entries of LDS
     __syncthreads();
     int wrun = 0;
     for (int base = 0; base < nw; base += VNEC_BLOCK) {
@@ -207,7 +211,7 @@ __global__ __launch_bounds__(VNEC_BLOCK) void k_win_layout(
     for (int d = tid; d < T; d += VNEC_BLOCK) {
         const int q = d / lw, jj = d % lw, k = q % nt, j = (q / nt) * lw + jj;
         const int i = k * ipt + j;
-        wl[sb + d] = i < nz ? lcol[(int64_t)c0.y + i] : (uint16_t)nec[t];
+        wl[sb + d] = i < nz ? lcol[(int64_t)c0.y + i] : (uint16_t)(nec[t] & ~VNEC_WIN_WIDE);
     }
 }
 
@@ -241,7 +245,7 @@ extern "C" int vnec_hip_win_desc(const int32_t *ptr, int64_t nrows, const int32_
     return (int)hipGetLastError();
 }
 
-extern "C" int vnec_hip_win_list(const int32_t *coords, int64_t ntiles, const int32_t *uniq, const int32_t *nec,
+extern "C" int vnec_hip_win_list(const int32_t *coords, int64_t ntiles, const int32_t *uniq, int32_t *nec,
                                  int32_t *wbase, uint16_t *woff, int32_t *wide, void *stream)
 {
     hipLaunchKernelGGL(k_win_list, dim3((unsigned)ntiles), dim3(VNEC_BLOCK), 0, (hipStream_t)stream,
@@ -364,7 +368,7 @@ __global__ __launch_bounds__(WIN_NT) void k_spmv_win(vnec_win_args a, int grid)
     const int t = (int)xcd_tile(blockIdx.x, grid);
     if (t >= a.ntiles) return;
     const int4 d0 = ((const int4 *)a.desc)[2 * t], d1 = ((const int4 *)a.desc)[2 * t + 1];
-    const int x0 = d0.x, y0 = d0.y, nrow = d0.z, nz = d0.w, nec = d1.x;
+    const int x0 = d0.x, y0 = d0.y, nrow = d0.z, nz = d0.w, nec = d1.x & ~VNEC_WIN_WIDE;
     F *s_x = (F *)s_raw;     // the x window and a zero for unused slots
     F *s_y = s_x + nec + 1;  // the tile's row sums
     F *s_pad = s_x + a.entries;
@@ -373,10 +377,10 @@ __global__ __launch_bounds__(WIN_NT) void k_spmv_win(vnec_win_args a, int grid)
     // the last one again
     uint32_t c[IPT];
     int cbv = 0;
-    {
+    const uint32_t last = nec - 1;
+    if (W16 && !(d1.x & VNEC_WIN_WIDE)) {
         const int64_t ch = (int64_t)(y0 >> 6) + t;
-        const uint32_t last = nec - 1;
-        if (W16 && nec > 0) {
+        if (nec > 0) {
             const uint32_t q = lane * NW + w;
             cbv = win_uniform(a.wbase + ch)[q < (last >> 6) ? q : (last >> 6)];
         }
@@ -385,9 +389,18 @@ __global__ __launch_bounds__(WIN_NT) void k_spmv_win(vnec_win_args a, int grid)
             if (g * WIN_NT < nec) {
 #pragma unroll
                 for (int u = g; u < g + 4; u++) {
-                    const uint32_t k = u * WIN_NT + tid, i = k < last ? k : last;
-                    c[u] = W16 ? (uint32_t)__builtin_nontemporal_load(win_uniform(a.woff + ch * 64) + i)
-                               : (uint32_t)__builtin_nontemporal_load(win_uniform(a.win + y0) + i);
+                    const uint32_t k = u * WIN_NT + tid;
+                    c[u] = __builtin_nontemporal_load(win_uniform(a.woff + ch * 64) + (k < last ? k : last));
+                }
+            }
+    } else {
+#pragma unroll
+        for (int g = 0; g < IPT; g += 4)
+            if (g * WIN_NT < nec) {
+#pragma unroll
+                for (int u = g; u < g + 4; u++) {
+                    const uint32_t k = u * WIN_NT + tid;
+                    c[u] = __builtin_nontemporal_load(win_uniform(a.win + y0) + (k < last ? k : last));
                 }
             }
     }
@@ -420,7 +433,7 @@ __global__ __launch_bounds__(WIN_NT) void k_spmv_win(vnec_win_args a, int grid)
         if (g * WIN_NT < nec) {
 #pragma unroll
             for (int u = g; u < g + 4; u++) {
-                if (W16) {
+                if (W16) {  // (x below 4 GiB: 32-bit byte offsets)
                     const WIN_GLOBAL char *xb =
                         (const WIN_GLOBAL char *)win_uniform(x + __builtin_amdgcn_readlane(cbv, u));
                     xv[u] = *(const WIN_GLOBAL F *)(xb + c[u] * (uint32_t)sizeof(F));

@@ -154,7 +154,8 @@ struct vnec_plan_s {
        names when w_threads > 0 (vnec_win_args describes the arrays) */
     int w_threads, w_ipt; /* threads per tile, items per thread          */
     int w_entries;        /* LDS entries of the largest tile             */
-    int64_t w_window;     /* window entries over all tiles               */
+    int64_t w_window, w_wide; /* window entries over all tiles, over those
+                                 read from 32-bit lists                  */
     double *w_val;
     float *w_hi, *w_lo;
     uint16_t *w_rank, *w_rbase, *w_off;

@@ -110,14 +110,15 @@ void vnec_window_release(struct vnec_plan_s *p)
  * start, and the tiles are that much shorter than T: fewer cut rows (a slot
  * that stays empty is not read).  T / 16, or T / 64 where that saves a round
  * of resident workgroups (R-MAT 18, 518 tiles of 7680 against 493 of 8064 on
- * 512 workgroups: 20.3 against 17.8 us; power-law rows 59.0 against 52.9). */
+ * 512 workgroups: 20.3 against 17.8 us; power-law rows 59.0 against 52.9; R-MAT
+ * 19 FP32, 794 against 757 on 768: 23.7 against 21.1). */
 static int window_snap(int64_t T, int64_t weight, int enc)
 {
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
         cus = 256;
-    const int64_t wgs = (int64_t)cus * (T > 4096 && enc != VNEC_ENC_FP32 ? 2 : 4);
+    const int64_t wgs = (int64_t)cus * (T <= 4096 ? 4 : enc == VNEC_ENC_FP32 ? 3 : 2);
     const int64_t s16 = T - T / 16, s64 = T - T / 64;
     const int64_t p16 = (weight + s16 - 1) / s16, p64 = (weight + s64 - 1) / s64;
     return (int)((p64 + wgs - 1) / wgs < (p16 + wgs - 1) / wgs ? T / 64 : T / 16);
@@ -128,8 +129,9 @@ static SpB_Info build_at(struct vnec_plan_s *p, const spb_csr *a, int ipt)
     hipStream_t s = vnec_stream();
     const int64_t T = VNEC_WIN_THREADS * (int64_t)ipt, nnz = p->nnz;
     const int enc = p->tune.encoding;
-    const int snap = window_snap(T, nnz + p->nrows * VNEC_WIN_ROW8 / 8, enc);
-    const int64_t step = T - snap, P = (nnz + p->nrows * VNEC_WIN_ROW8 / 8 + step - 1) / step;
+    const int snap = window_snap(T, p->nnz + p->nrows * VNEC_WIN_ROW8 / 8, enc);
+    const int64_t weight = nnz + p->nrows * VNEC_WIN_ROW8 / 8, P = (weight + T - snap - 1) / (T - snap);
+    const int64_t step = (weight + P - 1) / P; /* equal tiles: no sparse last one */
     const size_t slots = (size_t)(P * T), esz = enc == VNEC_ENC_FP32 ? sizeof(float) : sizeof(double);
     const size_t words = (size_t)(p->nrows / 64 + P + 1), chunks = (size_t)(nnz / 64 + P + 1);
     int64_t bytes = 0;
@@ -152,7 +154,7 @@ static SpB_Info build_at(struct vnec_plan_s *p, const spb_csr *a, int ipt)
     int32_t *tmp = (int32_t *)vnec_malloc_dev(sizeof(int32_t) * (size_t)(2 * P + 2), NULL);
     uint16_t *lcol = (uint16_t *)vnec_malloc_dev(sizeof(uint16_t) * (size_t)nnz, NULL);
     int32_t *nec = tmp, *nsum = tmp + P, *mx_dev = tmp + 2 * P;
-    int32_t mx[2] = {0, 0}; /* LDS entries; whether a distance passes 16 bits */
+    int32_t mx[2] = {0, 0}; /* LDS entries; whether a tile is wide */
     int32_t *hnec = (int32_t *)malloc(sizeof(int32_t) * (size_t)P);
     SpB_Info rc = p->coords && p->carry && p->w_desc && p->w_win && p->w_base && p->w_off &&
                           (enc == VNEC_ENC_FP64 ? (void *)p->w_val : (void *)p->w_hi) &&
@@ -165,12 +167,12 @@ static SpB_Info build_at(struct vnec_plan_s *p, const spb_csr *a, int ipt)
     if (rc == SpB_SUCCESS) /* (nsum: scratch for the run counts) */
         rc = vnec_hip_ok(vnec_hip_ecr_tiles_pass1(p->col, p->coords, P, lcol, NULL, p->w_win, nec, nsum, s),
                          "windows");
-    if (rc == SpB_SUCCESS)
-        rc = vnec_hip_ok(vnec_hip_win_desc(a->d_ptr, p->nrows, p->coords, P, nec, p->w_desc, s), "window rows");
     if (rc == SpB_SUCCESS) rc = vnec_hip_ok(hipMemsetAsync(mx_dev, 0, sizeof mx, s), "memset");
     if (rc == SpB_SUCCESS)
         rc = vnec_hip_ok(vnec_hip_win_list(p->coords, P, p->w_win, nec, p->w_base, p->w_off, mx_dev + 1, s),
                          "window lists");
+    if (rc == SpB_SUCCESS)
+        rc = vnec_hip_ok(vnec_hip_win_desc(a->d_ptr, p->nrows, p->coords, P, nec, p->w_desc, s), "window rows");
     if (rc == SpB_SUCCESS)
         rc = vnec_hip_ok(vnec_hip_win_layout(a->d_ptr, a->d_val, lcol, p->coords, P, ipt, enc, p->w_val, p->w_hi,
                                              p->w_lo, p->w_rank, p->w_flags, p->w_rmask, p->w_rbase, nec, nsum,
@@ -184,17 +186,26 @@ static SpB_Info build_at(struct vnec_plan_s *p, const spb_csr *a, int ipt)
     vnec_free_dev(lcol);
     if (rc == SpB_SUCCESS) {
         p->w_window = 0;
-        for (int64_t t = 0; t < P; t++) p->w_window += hnec[t];
+        int64_t wide = 0; /* entries of the tiles read from the 32-bit lists */
+        for (int64_t t = 0; t < P; t++) {
+            p->w_window += hnec[t] & ~VNEC_WIN_WIDE;
+            if (hnec[t] & VNEC_WIN_WIDE) wide += hnec[t] & ~VNEC_WIN_WIDE;
+        }
         p->w_entries = mx[0];
-        if (mx[1]) {
+        p->w_wide = wide;
+        if (!mx[1]) {
+            vnec_free_dev(p->w_win);
+            p->w_win = NULL;
+        } else {
+            bytes += (int64_t)sizeof(int32_t) * nnz;
+        }
+        if (mx[1] && p->ncols * (int64_t)esz >= ((int64_t)1 << 32)) { /* 32-bit lists throughout */
             vnec_free_dev(p->w_base);
             vnec_free_dev(p->w_off);
             p->w_base = NULL;
             p->w_off = NULL;
-            bytes += (int64_t)sizeof(int32_t) * nnz;
+            p->w_wide = p->w_window;
         } else {
-            vnec_free_dev(p->w_win);
-            p->w_win = NULL;
             bytes += (int64_t)((sizeof(int32_t) + 64 * sizeof(uint16_t)) * chunks);
         }
         if (ipt > 8 && (size_t)(p->w_entries + 1) * esz > WINDOW_LDS_TWO) {
@@ -234,7 +245,7 @@ int64_t vnec_window_bytes(const struct vnec_plan_s *p)
     const int64_t vb = enc == VNEC_ENC_HI || enc == VNEC_ENC_FP32 ? 4 : 8, P = p->ntiles;
     /* values and ranks, the window's columns, the threads' flags, the row
      * masks and the tile descriptors */
-    return p->nnz * (vb + 2) + p->w_window * (p->w_off ? 2 : 4) + (p->w_off ? p->w_window / 16 : 0) +
+    return p->nnz * (vb + 2) + 2 * p->w_window + 2 * p->w_wide + p->w_window / 16 +
            4 * (p->nnz + p->w_ipt - 1) / p->w_ipt + 10 * (p->nrows / 64 + P) + 32 * P;
 }
 
