@@ -149,29 +149,29 @@ extern "C" int vnec_hip_scan_excl_i32(const int32_t *in, int32_t *out, int64_t n
 // tile's distinct columns (spmv_vnec_D_for_mxv.c:292-319 computes the same
 // ranks with dense flags).  Runs of consecutive distinct columns are
 // counted for the compact window description.
-template <int CAP>
-__global__ __launch_bounds__(VNEC_BLOCK) void k_ecr_tile_pass1(
+template <int CAP, int NT>
+__global__ __launch_bounds__(NT) void k_ecr_tile_pass1(
     const int32_t *__restrict__ col, const int2 *__restrict__ coords, int64_t ntiles,
     uint16_t *__restrict__ lcol16, int32_t *__restrict__ ecr32, int32_t *__restrict__ uniq,
     int32_t *__restrict__ nec, int32_t *__restrict__ nruns)
 {
     __shared__ uint32_t s_key[CAP];
     __shared__ uint16_t s_idx[CAP];
-    __shared__ int s_tmp[VNEC_NWAVES + 1];
+    __shared__ int s_tmp[NT / VNEC_WAVE + 1];
     int64_t t = blockIdx.x;
     if (t >= ntiles) return;
     int y0 = coords[t].y, y1 = coords[t + 1].y;
     int n = y1 - y0;
     int n2 = 1;
     while (n2 < n) n2 <<= 1;
-    for (int k = threadIdx.x; k < n2; k += VNEC_BLOCK) {
+    for (int k = threadIdx.x; k < n2; k += NT) {
         s_key[k] = k < n ? (uint32_t)col[y0 + k] : 0xFFFFFFFFu;
         s_idx[k] = (uint16_t)k;
     }
     __syncthreads();
     for (int k = 2; k <= n2; k <<= 1) {
         for (int j = k >> 1; j > 0; j >>= 1) {
-            for (int i = threadIdx.x; i < n2; i += VNEC_BLOCK) {
+            for (int i = threadIdx.x; i < n2; i += NT) {
                 int ixj = i ^ j;
                 if (ixj > i) {
                     bool up = (i & k) == 0;
@@ -189,7 +189,7 @@ __global__ __launch_bounds__(VNEC_BLOCK) void k_ecr_tile_pass1(
         }
     }
     int uniq_base = 0, run_base = 0;
-    for (int base = 0; base < n; base += VNEC_BLOCK) {
+    for (int base = 0; base < n; base += NT) {
         int k = base + threadIdx.x;
         int f = 0, g = 0;
         uint32_t key = 0;
@@ -199,8 +199,8 @@ __global__ __launch_bounds__(VNEC_BLOCK) void k_ecr_tile_pass1(
             g = f && ((k == 0) || (key != s_key[k - 1] + 1u));
         }
         int totf, totg;
-        int exf = block_excl_scan_i32(f, s_tmp, &totf);
-        block_excl_scan_i32(g, s_tmp, &totg);
+        int exf = block_excl_scan_i32<NT / VNEC_WAVE>(f, s_tmp, &totf);
+        block_excl_scan_i32<NT / VNEC_WAVE>(g, s_tmp, &totg);
         if (k < n) {
             int rank = uniq_base + exf + f - 1;
             int pos = y0 + s_idx[k];
@@ -255,13 +255,12 @@ extern "C" int vnec_hip_ecr_tiles_pass1(const int32_t *col, const int32_t *coord
     if (rc) return rc;
     if (mx > VNEC_ECR_TILE_MAX_BIG) return (int)hipErrorInvalidValue;
     if (mx <= VNEC_ECR_TILE_MAX)
-        hipLaunchKernelGGL(k_ecr_tile_pass1<VNEC_ECR_TILE_MAX>, dim3((unsigned)ntiles), dim3(VNEC_BLOCK),
+        hipLaunchKernelGGL((k_ecr_tile_pass1<VNEC_ECR_TILE_MAX, 256>), dim3((unsigned)ntiles), dim3(256),
                            0, (hipStream_t)stream, col, (const int2 *)coords, ntiles, lcol16, ecr32,
                            uniq, nec, nruns);
     else
-        hipLaunchKernelGGL(k_ecr_tile_pass1<VNEC_ECR_TILE_MAX_BIG>, dim3((unsigned)ntiles),
-                           dim3(VNEC_BLOCK), 0, (hipStream_t)stream, col, (const int2 *)coords, ntiles,
-                           lcol16, ecr32, uniq, nec, nruns);
+        hipLaunchKernelGGL((k_ecr_tile_pass1<VNEC_ECR_TILE_MAX_BIG, 1024>), dim3((unsigned)ntiles), dim3(1024), 0,
+                           (hipStream_t)stream, col, (const int2 *)coords, ntiles, lcol16, ecr32, uniq, nec, nruns);
     return (int)hipGetLastError();
 }
 
