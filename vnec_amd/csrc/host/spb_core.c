@@ -71,6 +71,7 @@ void *vnec_malloc_dev(size_t bytes, int64_t *acct)
     void *p = NULL;
     if (bytes == 0) bytes = 16;
     if (hipMalloc(&p, bytes) != hipSuccess) {
+        (void)hipGetLastError(); /* not the next launch's error */
         vnec_fail("hipMalloc(%zu) failed", bytes);
         return NULL;
     }

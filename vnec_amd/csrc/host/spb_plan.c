@@ -729,9 +729,12 @@ static SpB_Info plan_build(vnec_plan *plan, const SpB_Matrix A, const vnec_tunin
 
 SpB_Info vnec_plan_build_ext(vnec_plan *plan, const SpB_Matrix A, const vnec_tuning *t)
 {
-    return plan_build(plan, A, t, !t || t->variant < 0);
+    return !t || t->variant < 0 ? vnec_plan_build_chosen(plan, A, t) : plan_build(plan, A, t, 0);
 }
 
+/* Windowed and stream tiles keep a copy of the matrix and need scratch to
+ * build it (up to 40 bytes a nonzero): where the device has no room for that,
+ * the kernel that reads the matrix in place. */
 SpB_Info vnec_plan_build_chosen(vnec_plan *plan, const SpB_Matrix A, const vnec_tuning *t)
 {
     if (plan_build(plan, A, t, 1) == SpB_SUCCESS) return SpB_SUCCESS;
