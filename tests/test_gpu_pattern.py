@@ -267,3 +267,33 @@ def test_g_x_at_any_alignment(name, m):
         dy.free()
         p.free()
         A.free()
+
+
+@pytest.mark.parametrize("enc", ["fp64", "hilo", "hi", "fp32"])
+@pytest.mark.parametrize("n,lengths", [(1500, range(1, 33)), (768 * 512 + 77, (1, 2, 7, 27))],
+                         ids=["every_length", "values_before_window"])
+def test_g_row_lengths(n, lengths, enc):
+    """Every pattern length — whole batches of 3 to 10 positions and what is
+    left over — and both orders of values and window, against the oracle."""
+    dt = np.float32 if enc == "fp32" else np.float64
+    for length in lengths:
+        print(f"pattern of {length}, {n} rows, {enc}", flush=True)
+        cnt = np.minimum(length, n - np.arange(n))
+        ptr = np.concatenate([[0], np.cumsum(cnt)]).astype(np.int64)
+        col = np.repeat(np.arange(n), cnt) + np.arange(ptr[-1]) - np.repeat(ptr[:-1], cnt)
+        m = g.from_pattern(n, n, ptr, col.astype(np.int32), seed=length)
+        val, x = m.val.astype(dt), m.x.astype(dt)
+        A = spb.Matrix.from_csr(n, n, ptr, m.col, val, dtype=dt)
+        p = spb.Plan(A, "G", encoding=enc)
+        dx, dy = spb.DeviceArray.from_array(x), spb.DeviceArray.from_array(np.full(n, np.nan, dt))
+        p.spmv_dev(dx.ptr, dy.ptr)
+        y = dy.to_array(dt, n)
+        ax, ref = O.spmv_abs(ptr, m.col, val.astype(np.float64), x.astype(np.float64))
+        if enc == "fp32":
+            ok, worst = O.check_rows_f32(y, O.spmv_serial_f32(ptr, m.col, val, x), ptr, ax)
+        else:
+            ok, worst = O.check_rows(y, ref, ax, 2.0 ** -23 if enc == "hi" else TOL)
+        assert ok, (length, worst)
+        p.free()
+        dx.free()
+        dy.free()

@@ -144,7 +144,13 @@ __device__ __forceinline__ void stage_window(const vnec_pattern_args &a, const F
 // WIN: the workgroup first stages its x window in LDS (a.wsize entries,
 // 16-byte loads), so the rows' x reads, each entry shared by up to L rows
 // of neighbouring slices, are LDS reads instead of L2 requests.
-template <int U, int ENC, bool WIN>
+// What bounds it: the slots' stream (27-point stencil of 2.1M rows: 77 us, 6.3
+// TB/s) and, below a few million slots or with short rows, the round trips of
+// a lane, since a lane sums its row alone: U positions are loaded together,
+// and the L % U last ones one after another.  U is the size with the fewest
+// round trips (pattern_batch).  PRE: the first U values are loaded before the
+// window is staged.
+template <int U, int ENC, bool WIN, bool PRE>
 __global__ __launch_bounds__(G_ROWS) void k_spmv_pattern(vnec_pattern_args a, int64_t grid)
 {
     typedef typename enc_real<ENC>::type F;
@@ -154,23 +160,30 @@ __global__ __launch_bounds__(G_ROWS) void k_spmv_pattern(vnec_pattern_args a, in
     const int64_t b = xcd_tile(blockIdx.x, grid);
     const int64_t r0 = b * G_ROWS;  // first row of the workgroup
     if (r0 >= a.nrows) return;       // whole workgroup
-    if (WIN) {
-        stage_window(a, x, r0, s_xw);
-        __syncthreads();
-    }
     const int64_t s = b * G_WAVES + wave_id();
-    if (s >= a.nslices) return;
     const int t = (int)threadIdx.x;  // local row
     const int64_t row = r0 + t;
     const bool live = row < a.nrows;
     const uint32_t m = live ? __builtin_nontemporal_load(a.masks + row) : 0u;
     const int64_t v = s * (int64_t)a.L * 64 + lane_id();  // slot (slice s, l = 0, this lane)
+    F vv[U];
+    if (WIN) {
+        if (PRE && s < a.nslices && U <= a.L) {
+#pragma unroll
+            for (int u = 0; u < U; u++) vv[u] = slot_value<ENC>(a, v + (int64_t)u * 64);
+        }
+        stage_window(a, x, r0, s_xw);
+        __syncthreads();
+    }
+    if (s >= a.nslices) return;
     F acc = 0;
     int l = 0;
     for (; l + U <= a.L; l += U) {
-        F vv[U], xv[U];
+        F xv[U];
+        if (!(WIN && PRE) || l > 0) {
 #pragma unroll
-        for (int u = 0; u < U; u++) vv[u] = slot_value<ENC>(a, v + (int64_t)(l + u) * 64);
+            for (int u = 0; u < U; u++) vv[u] = slot_value<ENC>(a, v + (int64_t)(l + u) * 64);
+        }
 #pragma unroll
         for (int u = 0; u < U; u++)
             xv[u] = ((m >> (l + u)) & 1u) ? (WIN ? s_xw[a.wpos[l + u] + t] : x[row + a.pat[l + u]]) : (F)0;
@@ -230,6 +243,50 @@ extern "C" int vnec_hip_pattern_fill(const int32_t *ptr, const double *val, cons
     return (int)hipGetLastError();
 }
 
+typedef void (*pattern_kernel_t)(vnec_pattern_args, int64_t);
+
+template <int U>
+static pattern_kernel_t pick_pattern(int enc, bool win, bool pre)
+{
+#define PK(E_)                                                                              \
+    if (enc == E_)                                                                          \
+        return !win ? k_spmv_pattern<U, E_, false, false>                                   \
+               : pre ? k_spmv_pattern<U, E_, true, true> : k_spmv_pattern<U, E_, true, false>;
+    PK(0) PK(1) PK(2) PK(VNEC_ENC_F32_K)
+#undef PK
+    return nullptr;
+}
+
+// Positions loaded together, 3 to 10: the fewest round trips, L / U batches
+// and L % U single loads (at 8 throughout and now: 27 positions, 0.11M rows
+// 7.6 -> 6.4 us; 31, 0.1M 8.8 -> 6.4; 3, 2.0M 19.2 -> 13.8; 5, 1.0M 13.3 -> 9.6).
+static int pattern_batch(int L)
+{
+    int u = 8;
+    for (int c = 10; c >= 3; c--)
+        if (L / c + L % c < L / u + L % u) u = c;
+    return u;
+}
+
+// The first values ahead of the window from this many workgroups on (three a
+// compute unit): 27 positions, 0.51M rows 20.6 -> 19.3 us, 2.1M 77.7 -> 76.9; 3,
+// 2.0M 15.5 -> 13.8; but 27, 0.26M rows of FP32 6.5 -> 6.9 and 0.11M 6.4 -> 6.9.
+#define PATTERN_PRE_BLOCKS 768
+
+static pattern_kernel_t pick_pattern(int u, int enc, bool win, bool pre)
+{
+    switch (u) {
+    case 3: return pick_pattern<3>(enc, win, pre);
+    case 4: return pick_pattern<4>(enc, win, pre);
+    case 5: return pick_pattern<5>(enc, win, pre);
+    case 6: return pick_pattern<6>(enc, win, pre);
+    case 7: return pick_pattern<7>(enc, win, pre);
+    case 9: return pick_pattern<9>(enc, win, pre);
+    case 10: return pick_pattern<10>(enc, win, pre);
+    default: return pick_pattern<8>(enc, win, pre);
+    }
+}
+
 extern "C" int vnec_hip_spmv_pattern(const vnec_pattern_args *a, void *stream)
 {
     if (a->nslices <= 0) return 0;
@@ -240,15 +297,7 @@ extern "C" int vnec_hip_spmv_pattern(const vnec_pattern_args *a, void *stream)
     if (a->wsize < 0 || a->wsize > VNEC_PATTERN_WIN_MAX || a->nwin < 0 || a->nwin > a->L)
         return (int)hipErrorInvalidValue;
     const bool win = a->wsize > 0;
-    void (*k)(vnec_pattern_args, int64_t) =
-        win ? (a->encoding == 0   ? k_spmv_pattern<8, 0, true>
-               : a->encoding == 1 ? k_spmv_pattern<8, 1, true>
-               : a->encoding == 2 ? k_spmv_pattern<8, 2, true>
-                                  : k_spmv_pattern<8, VNEC_ENC_F32_K, true>)
-            : (a->encoding == 0   ? k_spmv_pattern<8, 0, false>
-               : a->encoding == 1 ? k_spmv_pattern<8, 1, false>
-               : a->encoding == 2 ? k_spmv_pattern<8, 2, false>
-                                  : k_spmv_pattern<8, VNEC_ENC_F32_K, false>);
+    pattern_kernel_t k = pick_pattern(pattern_batch(a->L), a->encoding, win, blocks >= PATTERN_PRE_BLOCKS);
     const size_t lds = win ? (a->encoding == VNEC_ENC_F32_K ? sizeof(float) : sizeof(double)) * (size_t)a->wsize : 0;
     hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(G_ROWS), lds, (hipStream_t)stream, *a, grid);
     return (int)hipGetLastError();
