@@ -200,3 +200,23 @@ def test_window_relabelled_columns_beyond_the_training_sizes():
     ok, worst = _check(m, dy.to_array(np.float64, m.nrows), "fp64")
     assert ok, (p.info(), worst)
     p.free()
+
+
+@pytest.mark.parametrize("n,hb,windowed", [(29999, 10, True), (30000, 10, False), (14425, 9, False)])
+def test_short_pattern_matrices_run_windowed_tiles(n, hb, windowed):
+    """Pattern matrices below 30000 rows of at least 20 entries: windowed tiles
+    under the learned mode's pick, pattern slices where they are named."""
+    m = g.banded(n, hb, seed=17)
+    A = spb.Matrix.from_csr(m.nrows, m.ncols, m.ptr, m.col, m.val)
+    p, q = spb.Plan(A, "learned"), spb.Plan(A, "G")
+    if p.info().variant == "G":
+        assert _windowed(p) == (windowed and m.nnz >= 20 * n)
+    assert not _windowed(q)
+    dx = spb.DeviceArray.from_array(m.x)
+    for plan in (p, q):
+        dy = spb.DeviceArray.from_array(np.full(m.nrows, np.nan))
+        plan.spmv_dev(dx.ptr, dy.ptr)
+        ok, worst = _check(m, dy.to_array(np.float64, m.nrows), "fp64")
+        assert ok, worst
+        dy.free()
+        plan.free()

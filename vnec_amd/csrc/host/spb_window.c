@@ -28,6 +28,14 @@ static int contiguous(const spb_csr *a)
  * 27.6 against 26.7).  FP32 slices never do (16.8M: 21.7-83 against 19.0-23). */
 #define WINDOW_SLICE_NNZ ((int64_t)15 << 20)
 
+/* Pattern slices read no columns at all, but a lane sums its row alone: below
+ * this many rows of this length most of the chip idles (27-point stencil, 4k
+ * rows: slices 4.4 us, windowed 3.6; 14k 5.5, 3.9; 30k 5.5, 4.5; 29-wide band of
+ * 14k rows 5.6, 3.9; but 32k rows of 31: 5.3, 5.3, 47k of 27: 5.6, 5.8, and 32k
+ * rows of 17: 4.0, 4.4). */
+#define WINDOW_PATTERN_ROWS 30000
+#define WINDOW_PATTERN_LEN 20
+
 int vnec_window_applies(const spb_csr *a, const vnec_tuning *t)
 {
     if (a->nnz == 0 || t->nrhs > 1) return 0;
@@ -39,7 +47,10 @@ int vnec_window_applies(const spb_csr *a, const vnec_tuning *t)
         return 1;
     case VNEC_VAR_S:
         return t->encoding == VNEC_ENC_FP32 || (int64_t)a->nnz < WINDOW_SLICE_NNZ || !contiguous(a);
-    default: /* pattern slices read no columns at all */
+    case VNEC_VAR_G:
+        return (int64_t)a->base.row < WINDOW_PATTERN_ROWS &&
+               (int64_t)a->nnz >= WINDOW_PATTERN_LEN * (int64_t)a->base.row;
+    default:
         return 0;
     }
 }
