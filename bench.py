@@ -265,7 +265,7 @@ def selection_label(spb, A, mode, info, k):
 
 def kernel_name(info, k, windowed=False):
     if windowed:
-        return "k_spmv_win"
+        return "k_spmv_win" if k == 1 else "k_spmm_tiles"
     if k > 1:
         return "k_spmv_mergeKg" if k >= 4 else "k_spmv_mergeK"
     if info.grid == -2:
