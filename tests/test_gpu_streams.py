@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 import oracle as O
-from test_gpu_window import _cut_rows, _empty_stretches, _repeated_descending, _rows, _windowed
+from test_gpu_window import _cut_rows, _empty_stretches, _large_x, _repeated_descending, _rows, _windowed
 from vnec_amd import matgen as g
 from vnec_amd import spb
 
@@ -101,3 +101,32 @@ def test_stream_tiles_unaligned_vectors_and_infinities(k):
         if not bad:
             first = y if first is None else first
             assert np.array_equal(y, first)
+
+
+@pytest.mark.parametrize("k", [2, 4, 8, 16])
+@pytest.mark.parametrize("gib", [3, 4], ids=["32_bit_offsets", "64_bit_offsets"])
+def test_stream_tiles_large_x(gib, k):
+    """x beyond 2 GiB, where an offset does not fit an int, and from 4 GiB on,
+    where it does not fit 32 bits: the same columns as in a small matrix, the
+    same bits."""
+    print(f"streams large x: {gib} GiB, k={k}", flush=True)
+    ncols = (gib << 30) // (8 * k) + 999
+    ptr, col, used, inv, val = _large_x(ncols)
+    xs = np.random.default_rng(k).uniform(-1, 1, (len(used), k))
+    y = []
+    for n, c in ((ncols, col), (len(used), inv)):
+        A = spb.Matrix.from_csr(len(ptr) - 1, n, ptr, c, val)
+        p = spb.Plan(A, "learned", nrhs=k)
+        assert _windowed(p)
+        dx, dy = spb.DeviceArray(8 * n * k), spb.DeviceArray.from_array(np.full((len(ptr) - 1) * k, np.nan))
+        for at, row in zip(used if n == ncols else range(n), xs):
+            spb.L.check(spb.L.load().vnec_memcpy_h2d_ext(dx.ptr + 8 * k * int(at), row.ctypes.data, row.nbytes), "h2d")
+        p.spmv_dev(dx.ptr, dy.ptr)
+        y.append(dy.to_array(np.float64, (len(ptr) - 1) * k))
+        for h in (p, dx, dy):
+            h.free()
+    assert np.array_equal(y[0].view(np.uint64), y[1].view(np.uint64))
+    for c in range(k):
+        ax, ref = O.spmv_abs(ptr, inv, val, np.ascontiguousarray(xs[:, c]))
+        ok, worst = O.check_rows(np.ascontiguousarray(y[0][c::k]), ref, ax, TOL)
+        assert ok, (c, worst)

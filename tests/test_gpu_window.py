@@ -79,6 +79,18 @@ def _mixed_wide():  # long rows of consecutive columns beside rows over eight mi
     return _rows(lens, 8_000_000, 14, cols=np.concatenate(cols))
 
 
+def _large_x(ncols):
+    """400 rows over the whole of ncols columns, the first and the last one
+    among them: row offsets, columns, the columns used, the columns' positions
+    among those, values."""
+    rng = np.random.default_rng(16)
+    col = rng.integers(0, ncols, 400 * 7)
+    col[[0, -1]] = 0, ncols - 1
+    used, inv = np.unique(col, return_inverse=True)
+    return (np.arange(0, len(col) + 1, 7), col.astype(np.int32), used, inv.astype(np.int32).ravel(),
+            rng.uniform(-1, 1, len(col)))
+
+
 MATRICES = {
     "one": lambda: _rows([1], 1, 1),
     "edge2047": lambda: _tile_edge(2047), "edge2048": lambda: _tile_edge(2048), "edge2049": lambda: _tile_edge(2049),
@@ -220,3 +232,32 @@ def test_short_pattern_matrices_run_windowed_tiles(n, hb, windowed):
         assert ok, worst
         dy.free()
         plan.free()
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+def test_windowed_large_x(dt):
+    """x of 4 GiB and more, whose tiles read 32-bit column lists throughout:
+    the same columns as in a small matrix, the same bits."""
+    ncols = (1 << 32) // np.dtype(dt).itemsize + 999
+    print(f"windowed large x: {ncols} columns, {np.dtype(dt)}", flush=True)
+    ptr, col, used, inv, val = _large_x(ncols)
+    n, xs = len(ptr) - 1, np.random.default_rng(1).uniform(-1, 1, len(used)).astype(dt)
+    y = []
+    for nc, c in ((ncols, col), (len(used), inv)):
+        A = spb.Matrix.from_csr(n, nc, ptr, c, val.astype(dt), dtype=dt)
+        p = spb.Plan(A, "learned")
+        assert _windowed(p)
+        dx, dy = spb.DeviceArray(xs.itemsize * nc), spb.DeviceArray.from_array(np.full(n, np.nan, dt))
+        for at, v in zip(used if nc == ncols else range(nc), xs.reshape(-1, 1)):
+            spb.L.check(spb.L.load().vnec_memcpy_h2d_ext(dx.ptr + xs.itemsize * int(at), v.ctypes.data, v.nbytes), "h2d")
+        p.spmv_dev(dx.ptr, dy.ptr)
+        y.append(dy.to_array(dt, n))
+        for h in (p, dx, dy):
+            h.free()
+    assert np.array_equal(y[0].view(np.uint8), y[1].view(np.uint8))
+    ax, ref = O.spmv_abs(ptr, inv, val.astype(dt).astype(np.float64), xs.astype(np.float64))
+    if dt == np.float32:
+        ok, worst = O.check_rows_f32(y[0], O.spmv_serial_f32(ptr, inv, val.astype(dt), xs), ptr, ax)
+    else:
+        ok, worst = O.check_rows(y[0], ref, ax, TOL["fp64"])
+    assert ok, worst

@@ -27,6 +27,7 @@
 #include "vnec_common.h"
 #include "vnec_hip.h"
 #include "vnec_meet.h"
+#include "vnec_offset.h"
 
 typedef double spmm_d2 __attribute__((ext_vector_type(2)));
 typedef int spmm_i4 __attribute__((ext_vector_type(4)));
@@ -174,7 +175,7 @@ struct spmm_gather {
         const int c = group_bcast<Q, S % (4 * Q) / 4>(C[S / (4 * Q)][S % 4]);
         const spmm_d2 *p;
         if (BIG) p = (const spmm_d2 *)(x + (int64_t)c * K + q * VW);
-        else p = (const spmm_d2 *)((const char *)x + (uint32_t)(c * (K * 8) + q * (VW * 8)));
+        else p = (const spmm_d2 *)((const char *)x + vnec_x_offset(c, K * 8, q, VW * 8));
 #pragma unroll
         for (int h = 0; h < VW / 2; h++) xv[0][h] = p[h];
         spmm_gather<K, R, BIG, S + 1, N - 1>::run(x, C, q, xv + 1);
