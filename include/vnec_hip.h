@@ -265,7 +265,7 @@ int vnec_hip_win_layout(const int32_t *ptr, const double *val, const uint16_t *l
                         int64_t ntiles, int ipt, int encoding, double *wv, float *whi, float *wlo, uint16_t *wl,
                         uint32_t *wt, uint64_t *rmask, uint16_t *rbase, const int32_t *nec, int32_t *nsum,
                         int32_t *max_dev, void *slot, void *stream);
-/* Lets the kernel of these arguments use the LDS it needs (once per plan). */
+/* Lets the kernel of these arguments use the LDS its largest tile needs. */
 int vnec_hip_win_prepare(const vnec_win_args *a);
 int vnec_hip_spmv_win(const vnec_win_args *a, void *stream);
 
@@ -297,7 +297,6 @@ typedef struct {
 int vnec_hip_spmm_layout(const int32_t *ptr, const int32_t *col, const double *val, const int32_t *coords,
                          int64_t ntiles, int k, int run, double *sv, int32_t *sc, uint32_t *sf, uint64_t *rmask,
                          int32_t *rbase, int32_t *nsum, int32_t *max_dev, double *slot, void *stream);
-int vnec_hip_spmm_prepare(const vnec_spmm_args *a);
 int vnec_hip_spmm_tiles(const vnec_spmm_args *a, void *stream);
 
 /* Gather-ceiling probe over a matrix's values and columns (nnz): with

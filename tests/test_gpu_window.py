@@ -261,3 +261,46 @@ def test_windowed_large_x(dt):
     else:
         ok, worst = O.check_rows(y[0], ref, ax, TOL["fp64"])
     assert ok, worst
+
+
+class _FuncAttributes(spb.C.Structure):  # hipFuncAttributes
+    _fields_ = [("binaryVersion", spb.C.c_int), ("cacheModeCA", spb.C.c_int), ("constSizeBytes", spb.C.c_size_t),
+                ("localSizeBytes", spb.C.c_size_t), ("maxDynamicSharedSizeBytes", spb.C.c_int),
+                ("maxThreadsPerBlock", spb.C.c_int), ("numRegs", spb.C.c_int), ("preferredShmemCarveout", spb.C.c_int),
+                ("ptxVersion", spb.C.c_int), ("sharedSizeBytes", spb.C.c_size_t)]
+
+
+def test_plans_of_one_kernel_keep_its_lds_limit():
+    """A plan with a small window, built while one with a large window of the
+    same kernel is alive, leaves the kernel's LDS limit and the first plan's
+    results alone."""
+    lib, hip = spb.L.load(), spb.C.CDLL("libamdhip64.so")
+
+    def limit():
+        a = _FuncAttributes()
+        kernel = spb.C.addressof(spb.C.c_char.in_dll(lib, "_Z10k_spmv_winILi16ELi0ELb1EEv13vnec_win_argsi"))
+        assert hip.hipFuncGetAttributes(spb.C.byref(a), spb.C.c_void_p(kernel)) == 0
+        return a.maxDynamicSharedSizeBytes
+
+    big = g.rmat(17, 12, seed=10)
+    n = 20011  # rows of 80 among 2000 columns, no two of them neighbours
+    cols = 2 * np.sort(np.random.default_rng(18).integers(0, 2000, (n, 80)), axis=1)
+    small = _rows([80] * n, 4000, 18, cols=cols.ravel())
+    A = spb.Matrix.from_csr(big.nrows, big.ncols, big.ptr, big.col, big.val)
+    p = spb.Plan(A, "learned")
+    dx, dy = spb.DeviceArray.from_array(big.x), spb.DeviceArray(8 * big.nrows)
+    p.spmv_dev(dx.ptr, dy.ptr)
+    want, before = dy.to_array(np.float64, big.nrows), limit()
+    B = spb.Matrix.from_csr(small.nrows, small.ncols, small.ptr, small.col, small.val)
+    q = spb.Plan(B, "learned")
+    for plan, m in ((p, big), (q, small)):  # 16 nonzeros a thread, both
+        assert _windowed(plan) and plan.info().ntiles < m.nnz / 4096
+    assert limit() == before >= 128 << 10
+    for run in (p.spmv_dev, p.spmv_graph, p.spmv_graph):
+        dy = spb.DeviceArray.from_array(np.full(big.nrows, np.nan))
+        run(dx.ptr, dy.ptr)
+        assert np.array_equal(dy.to_array(np.float64, big.nrows).view(np.uint64), want.view(np.uint64))
+    dx, dy = spb.DeviceArray.from_array(small.x), spb.DeviceArray(8 * small.nrows)
+    q.spmv_dev(dx.ptr, dy.ptr)
+    ok, worst = _check(small, dy.to_array(np.float64, small.nrows), "fp64")
+    assert ok, worst

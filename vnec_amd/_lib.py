@@ -207,7 +207,6 @@ SIGNATURES = {
     "vnec_hip_win_prepare": (C.c_int, [vp]),
     "vnec_hip_spmv_win": (C.c_int, [vp, vp]),
     "vnec_hip_spmm_layout": (C.c_int, [vp, vp, vp, vp, i64, C.c_int, C.c_int] + [vp] * 9),
-    "vnec_hip_spmm_prepare": (C.c_int, [vp]),
     "vnec_hip_spmm_tiles": (C.c_int, [vp, vp]),
     "vnec_hip_stream_grid": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int)]),
     "vnec_hip_stream_supported": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int]),

@@ -325,21 +325,14 @@ static spmm_kernel_t pick_spmm(int k, int run, bool big)
 
 static size_t spmm_lds(const vnec_spmm_args *a) { return (size_t)a->sums * a->k * sizeof(double); }
 
-extern "C" int vnec_hip_spmm_prepare(const vnec_spmm_args *a)
-{
-    for (int big = 0; big < 2; big++) {
-        spmm_kernel_t k = pick_spmm(a->k, a->run, big);
-        if (!k) return (int)hipErrorInvalidValue;
-        hipError_t e = hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)spmm_lds(a));
-        if (e != hipSuccess) return (int)e;
-    }
-    return 0;
-}
+// Row sums of a tile take 33 KiB at most (k = 8, streams of 32: 521 of them), below
+// what every kernel may use without asking.
+#define SPMM_LDS_MAX (40 * 1024)
 
 extern "C" int vnec_hip_spmm_tiles(const vnec_spmm_args *a, void *stream)
 {
     spmm_kernel_t k = pick_spmm(a->k, a->run, a->ncols * a->k * 8 >= ((int64_t)1 << 32));
-    if (!k || (((uintptr_t)a->x | (a->ldy ? 0 : (uintptr_t)a->y)) & 15)) return (int)hipErrorInvalidValue;
+    if (!k || spmm_lds(a) > SPMM_LDS_MAX || (((uintptr_t)a->x | (a->ldy ? 0 : (uintptr_t)a->y)) & 15)) return (int)hipErrorInvalidValue;
     if (a->ntiles <= 0) return 0;
     const int64_t grid = xcd_grid(a->ntiles);
     hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(VNEC_BLOCK), spmm_lds(a), (hipStream_t)stream, *a, (int)grid);

@@ -550,17 +550,26 @@ static size_t win_lds(const vnec_win_args *a)
     return (size_t)(a->entries + 1) * (a->encoding == VNEC_ENC_F32_K ? sizeof(float) : sizeof(double));
 }
 
+// The most a tile of this kernel can need: its nonzeros all in columns of
+// their own and each a row's last.
+static size_t win_lds_max(const vnec_win_args *a)
+{
+    return (size_t)(2 * WIN_NT * a->ipt + 2) * (a->encoding == VNEC_ENC_F32_K ? sizeof(float) : sizeof(double));
+}
+
+// The limit is the kernel's, not the plan's: the same value whichever plan
+// asks, so that no plan lowers it under another one's launches.
 extern "C" int vnec_hip_win_prepare(const vnec_win_args *a)
 {
     win_kernel_t k = pick_win(a->ipt, a->encoding, a->woff != nullptr);
     if (!k) return (int)hipErrorInvalidValue;
-    return (int)hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)win_lds(a));
+    return (int)hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)win_lds_max(a));
 }
 
 extern "C" int vnec_hip_spmv_win(const vnec_win_args *a, void *stream)
 {
     win_kernel_t k = pick_win(a->ipt, a->encoding, a->woff != nullptr);
-    if (!k) return (int)hipErrorInvalidValue;
+    if (!k || win_lds(a) > win_lds_max(a)) return (int)hipErrorInvalidValue;
     if (a->ntiles <= 0) return 0;
     const int64_t grid = xcd_grid(a->ntiles);
     hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(WIN_NT), win_lds(a), (hipStream_t)stream, *a, (int)grid);

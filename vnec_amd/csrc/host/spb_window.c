@@ -361,14 +361,6 @@ SpB_Info vnec_streams_build(struct vnec_plan_s *p, const spb_csr *a)
     if (rc == SpB_SUCCESS) rc = vnec_hip_ok(hipMemcpyAsync(&mx, mx_dev, sizeof mx, hipMemcpyDeviceToHost, s), "d2h");
     if (rc == SpB_SUCCESS) rc = vnec_hip_ok(hipStreamSynchronize(s), "stream sync");
     vnec_free_dev(co);
-    if (rc == SpB_SUCCESS) {
-        vnec_spmm_args m;
-        memset(&m, 0, sizeof m);
-        m.k = k;
-        m.run = run;
-        m.sums = mx;
-        rc = vnec_hip_ok(vnec_hip_spmm_prepare(&m), "stream LDS");
-    }
     p->m_ntiles = P;
     p->m_run = run;
     p->m_sums = mx;
