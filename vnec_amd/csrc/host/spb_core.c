@@ -16,6 +16,7 @@
 
 /* ---------------------------------------------------------------- errors */
 static __thread char g_err[512];
+static __thread int g_no_memory; /* see vnec_no_memory */
 
 const char *vnec_last_error(void) { return g_err; }
 
@@ -30,9 +31,12 @@ SpB_Info vnec_fail(const char *fmt, ...)
     return SpB_FAILURE;
 }
 
+int *vnec_no_memory(void) { return &g_no_memory; }
+
 SpB_Info vnec_hip_ok(int rc, const char *what)
 {
     if (rc == 0) return SpB_SUCCESS;
+    if (rc == hipErrorOutOfMemory) g_no_memory = 1;
     return vnec_fail("%s: HIP error %d (%s)", what, rc, hipGetErrorString((hipError_t)rc));
 }
 
@@ -72,6 +76,7 @@ void *vnec_malloc_dev(size_t bytes, int64_t *acct)
     if (bytes == 0) bytes = 16;
     if (hipMalloc(&p, bytes) != hipSuccess) {
         (void)hipGetLastError(); /* not the next launch's error */
+        g_no_memory = 1;
         vnec_fail("hipMalloc(%zu) failed", bytes);
         return NULL;
     }

@@ -201,6 +201,9 @@ SpB_Info vnec_fail(const char *fmt, ...);
  * IRD_VNEC) clear the error slot first, so vnec_last_error() afterwards
  * describes that call. */
 void vnec_clear_error(void);
+/* The calling thread's flag that device memory ran out, set by
+ * vnec_malloc_dev and vnec_hip_ok, cleared by who asks. */
+int *vnec_no_memory(void);
 SpB_Info vnec_hip_ok(int rc, const char *what);
 int vnec_runtime_ready(void);
 void *vnec_malloc_dev(size_t bytes, int64_t *acct);

@@ -733,11 +733,17 @@ SpB_Info vnec_plan_build_ext(vnec_plan *plan, const SpB_Matrix A, const vnec_tun
 }
 
 /* Windowed and stream tiles keep a copy of the matrix and need scratch to
- * build it (up to 40 bytes a nonzero): where the device has no room for that,
- * the kernel that reads the matrix in place. */
+ * build it (FP64 windowed tiles: 12 bytes a nonzero kept and 8 more while
+ * building, stream tiles 12; and a row takes the slots of 1/8 nonzero, with
+ * stream tiles of 4, or 8 at 16 right-hand sides): where the device has no
+ * room for that, the kernel that reads the matrix in place.  Any other failure
+ * is the caller's to see. */
 SpB_Info vnec_plan_build_chosen(vnec_plan *plan, const SpB_Matrix A, const vnec_tuning *t)
 {
+    int *no_memory = vnec_no_memory();
+    *no_memory = 0;
     if (plan_build(plan, A, t, 1) == SpB_SUCCESS) return SpB_SUCCESS;
+    if (!*no_memory) return SpB_FAILURE;
     vnec_clear_error();
     return plan_build(plan, A, t, 0);
 }
