@@ -101,16 +101,17 @@ typedef enum {
 } vnec_encoding;
 
 /* Negative vnec_tuning.variant values: how the plan chooses its variant,
- * tile granularity and schedule.  A plan the learned or autotune mode, an FP32
+ * tile granularity and schedule.  A plan that the learned mode, an FP32
  * selection or a Build_VNEC_* call chose runs as windowed tiles (distinct x
- * entries of a tile gathered into LDS once) where those are the faster form of
- * what it picked; vnec_plan_info_ext still reports the pick, with the windowed
- * tiles' count. */
+ * entries of a tile gathered into LDS once) by a rule on its pick, a plan of
+ * the autotune mode where they were the fastest it timed; vnec_plan_info_ext
+ * still reports the pick, with the windowed tiles' count. */
 typedef enum {
     VNEC_SELECT_LEARNED = -1,   /* the trained MLP over matrix statistics (the
                                    rule below when no model is installed)    */
     VNEC_SELECT_AUTOTUNE = -2,  /* exhaustive: build and time every candidate
-                                   (FP32 matrices: every FP32 plan shape)    */
+                                   (FP32 matrices: every FP32 plan shape) and
+                                   windowed tiles beside the fastest         */
     VNEC_SELECT_RULE = -3,      /* S when 64-row slice padding <= 1.15, else
                                    persistent L at 7 items per thread        */
     VNEC_SELECT_REFERENCE = -4, /* the reference dispatch (nrows >= 3e6: L;

@@ -87,3 +87,21 @@ def test_other_failures_reach_the_caller(stub, nrhs):
     _plant(stub, layout_error=719)
     with pytest.raises(RuntimeError, match="layout: HIP error 719"):
         spb.Plan(A, "learned", nrhs=nrhs)
+
+
+@pytest.mark.parametrize("win_us,other_us", [(9.0, 5.0), (5.0, 9.0)], ids=["named_faster", "windowed_faster"])
+@pytest.mark.parametrize("enc", ["fp64", "hilo", "hi", "fp32"])
+def test_autotune_keeps_the_fastest_it_timed(stub, enc, win_us, other_us):
+    """The autotune mode times windowed tiles beside the named shapes and runs
+    whichever was faster, also from the cached comparison."""
+    A = _matrix(np.float32 if enc == "fp32" else np.float64)
+    _plant(stub, win_us=win_us, other_us=other_us)
+    for _ in range(2):
+        p = spb.Plan(A, "autotune", encoding=enc)
+        launches = [C.c_int.in_dll(stub, "stub_" + k).value for k in ("win_launches", "other_launches")]
+        assert min(launches) > 0, "both were timed"
+        assert _windowed(p) == (win_us < other_us)
+        x, y = spb.DeviceArray(8 * A.ncols), spb.DeviceArray(8 * A.nrows)
+        assert p.time(x.ptr, y.ptr, 20) == pytest.approx(min(win_us, other_us) * 1e-3)
+        for h in (p, x, y):
+            h.free()

@@ -194,6 +194,7 @@ static void matrix_drop_device(spb_csr *a)
     a->pattern_ready = 0;
     a->refined_slice_ipt = 0;
     a->window_relabel = 0;
+    memset(a->tuned_window, 0, sizeof a->tuned_window);
 }
 
 SpB_Info SpB_Matrix_free(SpB_Matrix *A)

@@ -450,9 +450,9 @@ int vnec_pattern_rule(spb_csr *a)
     return (double)nreg >= 0.9 * (double)a->base.row && (double)a->nnz >= 0.8 * slots;
 }
 
-/* t's plan; with windowed != 0 it may run as windowed tiles where they
- * apply (spb_window.c): the modes that choose a plan ask for that, a caller
- * that names a plan shape gets that shape. */
+/* t's plan; with windowed = 1 it may run as windowed tiles where they apply
+ * (spb_window.c): the modes that choose a plan ask for that, a caller that
+ * names a plan shape gets that shape; with windowed = 2 it does. */
 static SpB_Info plan_build(vnec_plan *plan, const SpB_Matrix A, const vnec_tuning *t, int windowed)
 {
     if (!plan) return vnec_fail("vnec_plan_build_ext: NULL plan handle");
@@ -464,6 +464,10 @@ static SpB_Info plan_build(vnec_plan *plan, const SpB_Matrix A, const vnec_tunin
     const int fp32 = a->base.element_type == SpB_FP32;
     if (fp32 && t && t->variant == VNEC_SELECT_AUTOTUNE) {
         if (vnec_autotune_fp32(a, &tune) != SpB_SUCCESS) return SpB_FAILURE;
+        if (windowed && a->nnz > 0) {
+            if (vnec_autotune_windowed(a, &tune, &tune, &windowed) != SpB_SUCCESS) return SpB_FAILURE;
+            windowed *= 2;
+        }
     } else if (fp32 && (!t || t->variant < 0)) {
         /* FP32 matrices (the selector's measurements are of the FP64
          * kernels): pattern slices where the pattern rule holds, else the
@@ -511,8 +515,15 @@ static SpB_Info plan_build(vnec_plan *plan, const SpB_Matrix A, const vnec_tunin
         }
         const int mode = t ? t->variant : VNEC_SELECT_LEARNED;
         if (mode != VNEC_SELECT_LEARNED && mode != VNEC_SELECT_AUTOTUNE) windowed = 0;
-        if (windowed && vnec_window_applies(a, &tune)) {
-            if (vnec_window_relabel(a, &tune) != SpB_SUCCESS) return SpB_FAILURE;
+        /* windowed tiles: the learned mode takes them where they apply, the
+         * autotune mode where they beat the fastest named shape */
+        const int compare = windowed && mode == VNEC_SELECT_AUTOTUNE && tune.nrhs == 1 && a->nnz > 0 &&
+                            tune.encoding >= 0 && tune.encoding < VNEC_ENC_N;
+        const int applies = windowed && !compare && vnec_window_applies(a, &tune);
+        vnec_tuning win = tune;
+        if ((compare || applies) && vnec_window_relabel(a, &win) != SpB_SUCCESS) return SpB_FAILURE;
+        if (applies) {
+            tune = win;
         } else if ((tune.variant == VNEC_VAR_L || tune.variant == VNEC_VAR_C) && tune.nrhs == 1 &&
             tune.encoding == VNEC_ENC_FP64) {
             /* CSR-ordered or column-sorted tiles, persistent or with
@@ -535,6 +546,11 @@ static SpB_Info plan_build(vnec_plan *plan, const SpB_Matrix A, const vnec_tunin
              * among the slice layouts is measured: 64-row slices or
              * pattern slices, whichever is faster */
             if (vnec_refine_slice_plan(a, &tune) != SpB_SUCCESS) return SpB_FAILURE;
+        }
+        if (compare) {
+            if (vnec_autotune_windowed(a, &tune, &win, &windowed) != SpB_SUCCESS) return SpB_FAILURE;
+            if (windowed) tune = win;
+            windowed *= 2;
         }
     }
     if (tune.nrhs <= 0) tune.nrhs = 1;
@@ -609,7 +625,7 @@ static SpB_Info plan_build(vnec_plan *plan, const SpB_Matrix A, const vnec_tunin
     }
     if (spb_matrix_upload(a) != SpB_SUCCESS) return SpB_FAILURE;
     const int streams = windowed && vnec_streams_apply(a, &tune);
-    windowed = windowed && vnec_window_applies(a, &tune);
+    windowed = windowed == 2 ? tune.nrhs == 1 && a->nnz > 0 : windowed && vnec_window_applies(a, &tune);
 
     struct vnec_plan_s *p = (struct vnec_plan_s *)calloc(1, sizeof *p);
     if (!p) return vnec_fail("out of memory");
@@ -730,6 +746,11 @@ static SpB_Info plan_build(vnec_plan *plan, const SpB_Matrix A, const vnec_tunin
 SpB_Info vnec_plan_build_ext(vnec_plan *plan, const SpB_Matrix A, const vnec_tuning *t)
 {
     return !t || t->variant < 0 ? vnec_plan_build_chosen(plan, A, t) : plan_build(plan, A, t, 0);
+}
+
+SpB_Info vnec_plan_build_windowed(vnec_plan *plan, const SpB_Matrix A, const vnec_tuning *t)
+{
+    return plan_build(plan, A, t, 2);
 }
 
 /* Windowed and stream tiles keep a copy of the matrix and need scratch to

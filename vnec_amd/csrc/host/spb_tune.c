@@ -270,6 +270,7 @@ SpB_Info vnec_autotune_ext(const SpB_Matrix A, int reps, double times_ms[VNEC_NC
     if (rc != SpB_SUCCESS) return rc;
     if (bi < 0) return vnec_fail("vnec_autotune_ext: no candidate applies");
     a->tuned_cand = bi;
+    memset(a->tuned_window, 0, sizeof a->tuned_window); /* compared with another pick */
     if (best) *best = bi;
     return SpB_SUCCESS;
 }
@@ -742,6 +743,33 @@ SpB_Info vnec_autotune_fp32(spb_csr *a, vnec_tuning *t)
     if (rc != SpB_SUCCESS) return rc;
     a->tuned_fp32 = bi;
     *t = FP32_SHAPES[bi];
+    return SpB_SUCCESS;
+}
+
+SpB_Info vnec_autotune_windowed(spb_csr *a, const vnec_tuning *t, const vnec_tuning *w, int *windowed)
+{
+    int *known = &a->tuned_window[t->encoding];
+    if (!*known) {
+        const int64_t nr = (int64_t)a->base.row, nc = (int64_t)a->base.col;
+        double *dx = (double *)vnec_malloc_dev(sizeof(double) * (size_t)(nc ? nc : 1), NULL);
+        double *dy = (double *)vnec_malloc_dev(sizeof(double) * (size_t)(nr ? nr : 1), NULL);
+        SpB_Info rc = dx && dy ? SpB_SUCCESS : SpB_FAILURE;
+        if (rc == SpB_SUCCESS) rc = vnec_hip_ok(vnec_hip_zero_f64(dx, nc, vnec_stream()), "zero x");
+        double named = INFINITY, win = INFINITY;
+        vnec_plan p = NULL;
+        if (rc == SpB_SUCCESS) rc = time_tuning(a, t, dx, dy, 20, &named);
+        if (rc == SpB_SUCCESS && vnec_plan_build_windowed(&p, (SpB_Matrix)a, w) == SpB_SUCCESS) {
+            rc = vnec_time_plan(p, dx, dy, 20, &win);
+            vnec_plan_free_ext(&p);
+        } else if (rc == SpB_SUCCESS) {
+            vnec_clear_error(); /* not a contender */
+        }
+        vnec_free_dev(dx);
+        vnec_free_dev(dy);
+        if (rc != SpB_SUCCESS) return rc;
+        *known = win < named ? 2 : 1;
+    }
+    *windowed = *known == 2;
     return SpB_SUCCESS;
 }
 
