@@ -110,8 +110,10 @@ typedef enum {
     VNEC_SELECT_LEARNED = -1,   /* the trained MLP over matrix statistics (the
                                    rule below when no model is installed)    */
     VNEC_SELECT_AUTOTUNE = -2,  /* exhaustive: build and time every candidate
-                                   (FP32 matrices: every FP32 plan shape) and
-                                   windowed tiles beside the fastest         */
+                                   (FP32 matrices: every FP32 plan shape;
+                                   several right-hand sides: granularities)
+                                   and windowed or stream tiles beside the
+                                   fastest                                   */
     VNEC_SELECT_RULE = -3,      /* S when 64-row slice padding <= 1.15, else
                                    persistent L at 7 items per thread        */
     VNEC_SELECT_REFERENCE = -4, /* the reference dispatch (nrows >= 3e6: L;

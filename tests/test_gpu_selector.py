@@ -231,14 +231,15 @@ def test_learned_mode_follows_compiled_model_on_held_out():
 
 @pytest.mark.parametrize("mode", ["autotune", "learned"])
 def test_multi_rhs_selection(mode):
-    """Several right-hand sides run the merge-path kernel; the autotuner
-    picks its granularity among the compiled ones."""
+    """Several right-hand sides: a merge-path plan, at 5 items per thread or
+    the granularity the autotuner measured fastest, for vectors that stream
+    tiles do not take."""
     k = 4
     m = g.rmat(12, 8, seed=45)
     A = _mat(m)
     p = spb.Plan(A, mode, nrhs=k)
     info = p.info()
-    assert info.variant == "L" and info.nrhs == k and info.ipt in (3, 5, 7)
+    assert info.variant == "L" and info.nrhs == k and info.ipt in ((3, 5, 7) if mode == "autotune" else (5,))
     X = np.random.default_rng(k).uniform(-1, 1, m.ncols * k)
     xv = spb.Vector.from_array(X)
     yv = spb.Vector(m.nrows * k)

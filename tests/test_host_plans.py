@@ -105,3 +105,22 @@ def test_autotune_keeps_the_fastest_it_timed(stub, enc, win_us, other_us):
         assert p.time(x.ptr, y.ptr, 20) == pytest.approx(min(win_us, other_us) * 1e-3)
         for h in (p, x, y):
             h.free()
+
+
+@pytest.mark.parametrize("tiles_us,kernel", [(9.0, "merge"), (2.0, "tiles")])
+@pytest.mark.parametrize("nrhs", [2, 4, 8, 16])
+def test_autotune_of_several_right_hand_sides(stub, nrhs, tiles_us, kernel):
+    """Stream tiles where they were faster than the merge-path kernel at its
+    best granularity; that granularity either way, since vectors aligned to 8
+    bytes only run it."""
+    A = _matrix()
+    _plant(stub, tiles_us=tiles_us)
+    (C.c_double * 16).in_dll(stub, "stub_merge_us")[3:8] = [3.0, 0, 6.0, 0, 5.0]
+    for _ in range(2):
+        p = spb.Plan(A, "autotune", nrhs=nrhs)
+        assert p.info().ipt == 3 and _windowed(p) == (kernel == "tiles")
+        x, y = (spb.DeviceArray(8 * (n * nrhs + 2)) for n in (A.ncols, A.nrows))
+        assert p.time(x.ptr, y.ptr, 20) == pytest.approx(min(tiles_us, 3.0) * 1e-3)
+        assert p.time(x.ptr + 8, y.ptr + 8, 20) == pytest.approx(3.0e-3)
+        for h in (p, x, y):
+            h.free()

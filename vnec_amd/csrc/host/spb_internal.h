@@ -63,8 +63,9 @@ typedef struct spb_csr {
     int refined_slice_variant, refined_slice_ipt_out;
     int window_relabel; /* windowed tiles faster over relabelled columns:
                            1 no, 2 yes (0: not measured)                */
-    int tuned_window[VNEC_ENC_N]; /* windowed tiles faster than the named
-                           shape of the autotune mode, per encoding: as above */
+    int tuned_window[VNEC_ENC_N + 4]; /* windowed tiles faster than the named
+                           shape of the autotune mode, per encoding, and stream
+                           tiles for 2, 4, 8 and 16 right-hand sides: as above */
     int feat_ready;     /* feat_ints holds the selector's statistics     */
     int pattern_ready;  /* pattern_rows holds the count below            */
     int64_t pattern_rows; /* rows that fit the dominant column-offset pattern */
@@ -235,7 +236,7 @@ double vnec_slice_padding(const spb_csr *a);
 /* As vnec_plan_build_ext, for a plan shape the library chose itself: it may
  * run as windowed tiles. */
 SpB_Info vnec_plan_build_chosen(vnec_plan *plan, const SpB_Matrix A, const vnec_tuning *t);
-/* As vnec_plan_build_ext, but as windowed tiles. */
+/* As vnec_plan_build_ext, but as windowed or stream tiles. */
 SpB_Info vnec_plan_build_windowed(vnec_plan *plan, const SpB_Matrix A, const vnec_tuning *t);
 
 /* ---- windowed tiles (spb_window.c) ---- */
@@ -299,8 +300,8 @@ SpB_Info vnec_refine_slice_plan(spb_csr *a, vnec_tuning *t);
  * merged column runs a workgroup's 256 rows read, staged in LDS when they
  * total at most VNEC_PATTERN_WIN_MAX entries (else wsize = 0). */
 void vnec_pattern_window(const int32_t *pat, int L, vnec_pattern_args *g);
-/* *windowed: whether windowed tiles of w beat the named shape t on a, both
- * timed as they run (cached on a until it changes or is autotuned again). */
+/* *windowed: whether windowed tiles of w (stream tiles for several right-hand
+ * sides) beat the named shape t on a, both timed as they run (cached on a until it changes or is autotuned again). */
 SpB_Info vnec_autotune_windowed(spb_csr *a, const vnec_tuning *t, const vnec_tuning *w, int *windowed);
 /* Best of three hipGraph-timed means of `iters` SpMVs of plan p. */
 SpB_Info vnec_time_plan(vnec_plan p, const void *dx, void *dy, int iters, double *ms_out);

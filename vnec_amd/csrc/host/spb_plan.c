@@ -497,10 +497,7 @@ static SpB_Info plan_build(vnec_plan *plan, const SpB_Matrix A, const vnec_tunin
         tune = g;
     } else {
         int nrhs = t && t->nrhs > 0 ? t->nrhs : 1;
-        int smode = t ? t->variant : VNEC_SELECT_LEARNED;
-        /* (stream tiles leave the merge-path kernel's granularity unused) */
-        if (nrhs > 1 && windowed && (!t || t->encoding == VNEC_ENC_FP64)) smode = VNEC_SELECT_LEARNED;
-        if (vnec_select_tuning(a, smode, nrhs, &tune) != SpB_SUCCESS)
+        if (vnec_select_tuning(a, t ? t->variant : VNEC_SELECT_LEARNED, nrhs, &tune) != SpB_SUCCESS)
             return SpB_FAILURE;
         if (t) tune.encoding = t->encoding;
         /* a candidate without a kernel for the requested encoding falls back
@@ -515,10 +512,12 @@ static SpB_Info plan_build(vnec_plan *plan, const SpB_Matrix A, const vnec_tunin
         }
         const int mode = t ? t->variant : VNEC_SELECT_LEARNED;
         if (mode != VNEC_SELECT_LEARNED && mode != VNEC_SELECT_AUTOTUNE) windowed = 0;
-        /* windowed tiles: the learned mode takes them where they apply, the
-         * autotune mode where they beat the fastest named shape */
-        const int compare = windowed && mode == VNEC_SELECT_AUTOTUNE && tune.nrhs == 1 && a->nnz > 0 &&
-                            tune.encoding >= 0 && tune.encoding < VNEC_ENC_N;
+        /* windowed tiles, and stream tiles for several right-hand sides: the
+         * learned mode takes them where they apply, the autotune mode where
+         * they beat the fastest named shape */
+        const int compare = windowed && mode == VNEC_SELECT_AUTOTUNE && a->nnz > 0 &&
+                            (tune.nrhs == 1 ? tune.encoding >= 0 && tune.encoding < VNEC_ENC_N
+                                            : vnec_streams_apply(a, &tune));
         const int applies = windowed && !compare && vnec_window_applies(a, &tune);
         vnec_tuning win = tune;
         if ((compare || applies) && vnec_window_relabel(a, &win) != SpB_SUCCESS) return SpB_FAILURE;

@@ -625,17 +625,16 @@ SpB_Info vnec_select_ext(const SpB_Matrix A, int mode, int *candidate)
  * per tile; the autotuner picks its granularity among the compiled ones. */
 static const int MULTI_IPT[] = {3, 5, 7};
 
+/* Launches per timing: four take 0.1 ms and more from 2^23 products on. */
+static int multi_iters(const spb_csr *a, int nrhs) { return (int64_t)a->nnz * nrhs >= (int64_t)1 << 23 ? 4 : 10; }
+
 static SpB_Info autotune_multi(spb_csr *a, int nrhs, int *ipt)
 {
     int64_t nr = (int64_t)a->base.row, nc = (int64_t)a->base.col;
-    size_t xb = sizeof(double) * (size_t)(nc * nrhs > 0 ? nc * nrhs : 1);
-    double *hx = (double *)malloc(xb);
-    double *dx = (double *)vnec_malloc_dev(xb, NULL);
+    double *dx = (double *)vnec_malloc_dev(sizeof(double) * (size_t)(nc * nrhs > 0 ? nc * nrhs : 1), NULL);
     double *dy = (double *)vnec_malloc_dev(sizeof(double) * (size_t)(nr * nrhs > 0 ? nr * nrhs : 1), NULL);
-    SpB_Info rc = (hx && dx && dy) ? SpB_SUCCESS : vnec_fail("out of memory");
-    for (int64_t i = 0; rc == SpB_SUCCESS && i < nc * nrhs; i++) hx[i] = 1.0 / (double)(1 + (i % 7));
-    if (rc == SpB_SUCCESS && nc)
-        rc = vnec_hip_ok(hipMemcpy(dx, hx, xb, hipMemcpyHostToDevice), "h2d");
+    SpB_Info rc = (dx && dy) ? SpB_SUCCESS : vnec_fail("out of memory");
+    if (rc == SpB_SUCCESS) rc = vnec_hip_ok(vnec_hip_zero_f64(dx, nc * nrhs, vnec_stream()), "zero x");
     double best = INFINITY;
     *ipt = 5;
     for (size_t c = 0; rc == SpB_SUCCESS && c < sizeof MULTI_IPT / sizeof MULTI_IPT[0]; c++) {
@@ -645,7 +644,7 @@ static SpB_Info autotune_multi(spb_csr *a, int nrhs, int *ipt)
         double tb = INFINITY;
         for (int r = 0; rc == SpB_SUCCESS && r < 3; r++) {
             double ms = 0.0;
-            rc = vnec_time_dev_ext(p, dx, dy, 10, 1, 0, &ms);
+            rc = vnec_time_dev_ext(p, dx, dy, multi_iters(a, nrhs), 1, 0, &ms);
             if (rc == SpB_SUCCESS && ms < tb) tb = ms;
         }
         vnec_plan_free_ext(&p);
@@ -654,7 +653,6 @@ static SpB_Info autotune_multi(spb_csr *a, int nrhs, int *ipt)
             *ipt = MULTI_IPT[c];
         }
     }
-    free(hx);
     vnec_free_dev(dx);
     vnec_free_dev(dy);
     return rc;
@@ -748,18 +746,20 @@ SpB_Info vnec_autotune_fp32(spb_csr *a, vnec_tuning *t)
 
 SpB_Info vnec_autotune_windowed(spb_csr *a, const vnec_tuning *t, const vnec_tuning *w, int *windowed)
 {
-    int *known = &a->tuned_window[t->encoding];
+    const int k = t->nrhs; /* 2, 4, 8 and 16 after the encodings */
+    int *known = &a->tuned_window[k == 1 ? t->encoding : VNEC_ENC_N + (k > 2) + (k > 4) + (k > 8)];
     if (!*known) {
-        const int64_t nr = (int64_t)a->base.row, nc = (int64_t)a->base.col;
+        const int64_t nr = (int64_t)a->base.row * k, nc = (int64_t)a->base.col * k;
+        const int iters = k == 1 ? 20 : multi_iters(a, k);
         double *dx = (double *)vnec_malloc_dev(sizeof(double) * (size_t)(nc ? nc : 1), NULL);
         double *dy = (double *)vnec_malloc_dev(sizeof(double) * (size_t)(nr ? nr : 1), NULL);
         SpB_Info rc = dx && dy ? SpB_SUCCESS : SpB_FAILURE;
         if (rc == SpB_SUCCESS) rc = vnec_hip_ok(vnec_hip_zero_f64(dx, nc, vnec_stream()), "zero x");
         double named = INFINITY, win = INFINITY;
         vnec_plan p = NULL;
-        if (rc == SpB_SUCCESS) rc = time_tuning(a, t, dx, dy, 20, &named);
+        if (rc == SpB_SUCCESS) rc = time_tuning(a, t, dx, dy, iters, &named);
         if (rc == SpB_SUCCESS && vnec_plan_build_windowed(&p, (SpB_Matrix)a, w) == SpB_SUCCESS) {
-            rc = vnec_time_plan(p, dx, dy, 20, &win);
+            rc = vnec_time_plan(p, dx, dy, iters, &win);
             vnec_plan_free_ext(&p);
         } else if (rc == SpB_SUCCESS) {
             vnec_clear_error(); /* not a contender */

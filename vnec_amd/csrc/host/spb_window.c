@@ -276,7 +276,7 @@ int vnec_plan_windowed(vnec_plan plan)
 SpB_Info vnec_window_relabel(spb_csr *a, vnec_tuning *t)
 {
     const int64_t nr = (int64_t)a->base.row, nc = (int64_t)a->base.col;
-    if ((t->variant != VNEC_VAR_L && t->variant != VNEC_VAR_C) || t->encoding != VNEC_ENC_FP64 ||
+    if ((t->variant != VNEC_VAR_L && t->variant != VNEC_VAR_C) || t->encoding != VNEC_ENC_FP64 || t->nrhs > 1 ||
         8 * nc < WINDOW_RELABEL_X || (int64_t)a->nnz <= WINDOW_RELABEL_NNZ)
         return SpB_SUCCESS;
     const int lanes = (t->lanes == 64 ? 0 : t->lanes) | VNEC_LANES_RELABEL;
