@@ -13,6 +13,7 @@ int stub_layout_error;            /* returned by the layout builders */
 int stub_choice;                  /* the learned selector's pick */
 double stub_win_us = 1, stub_tiles_us = 1, stub_merge_us[16], stub_other_us = 1;
 int stub_win_launches, stub_other_launches;
+int stub_x_changes;               /* windowed launches on another x than the one before */
 
 static double now_us, captured_us;
 static int capturing;
@@ -108,7 +109,13 @@ int vnec_hip_spmm_layout(const int32_t *ptr, const int32_t *col, const double *v
     return stub_layout_error;
 }
 
-int vnec_hip_spmv_win(const vnec_win_args *a, void *s) { return launch(stub_win_us, 1); }
+int vnec_hip_spmv_win(const vnec_win_args *a, void *s)
+{
+    static const double *last;
+    stub_x_changes += last != a->x;
+    last = a->x;
+    return launch(stub_win_us, 1);
+}
 int vnec_hip_spmm_tiles(const vnec_spmm_args *a, void *s) { return launch(stub_tiles_us, 1); }
 int vnec_hip_spmv_merge(const vnec_merge_args *m, void *s)
 {

@@ -51,7 +51,7 @@ def stub(stub_path, monkeypatch):
 
 def _plant(lib, **values):
     for name, v in {"largest": C.c_size_t(-1).value, "layout_error": 0, "choice": 4, "win_us": 1.0, "tiles_us": 1.0,
-                    "other_us": 1.0, "win_launches": 0, "other_launches": 0, **values}.items():
+                    "other_us": 1.0, "win_launches": 0, "other_launches": 0, "x_changes": 0, **values}.items():
         t = C.c_size_t if name == "largest" else C.c_double if name.endswith("us") else C.c_int
         t.in_dll(lib, "stub_" + name).value = v
 
@@ -124,3 +124,19 @@ def test_autotune_of_several_right_hand_sides(stub, nrhs, tiles_us, kernel):
         assert p.time(x.ptr + 8, y.ptr + 8, 20) == pytest.approx(3.0e-3)
         for h in (p, x, y):
             h.free()
+
+
+def test_kernel_times_of_relabelled_windowed_tiles_read_the_permuted_x(stub):
+    A = _matrix()
+    _plant(stub)
+    t = L.Tuning(spb.VNEC_VAR["L"], 7, spb.LANES_RELABEL, spb.VNEC_ENC["fp64"], 1, -1)
+    h = C.c_void_p()
+    stub.vnec_plan_build_windowed.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p]
+    L.check(stub.vnec_plan_build_windowed(C.byref(h), A.h, C.byref(t)), "build")
+    x, y = spb.DeviceArray(8 * A.ncols), spb.DeviceArray(8 * A.nrows)
+    L.check(stub.vnec_spmv_dev_ext(h, x.ptr, y.ptr), "SpMV")
+    a, b = C.c_double(), C.c_double()
+    _plant(stub)
+    L.check(stub.vnec_time_kernels_ext(h, x.ptr, y.ptr, 5, C.byref(a), C.byref(b)), "time")
+    assert C.c_int.in_dll(stub, "stub_win_launches").value == 7 and C.c_int.in_dll(stub, "stub_x_changes").value == 0
+    L.check(stub.vnec_plan_free_ext(C.byref(h)), "free")

@@ -22,7 +22,8 @@ static __global__ void k_meet_empty(int64_t n, int fp32, void *__restrict__ slot
 // in the slot and is done; the second takes it, empties the slot for the next
 // launch and goes on with the total.  The tree fixes the order of the sums,
 // one atomic exchange carries both the value and its arrival, and nothing is
-// waited for.
+// waited for.  Launches that share slots must follow one another, and each run
+// to its end: every entry of the library puts a plan's on its one stream.
 __device__ __forceinline__ bool meet_swap(double *slot, double &s)
 {
     typedef unsigned long long u64;

@@ -1279,9 +1279,10 @@ SpB_Info vnec_time_dev_ext(vnec_plan plan, const void *x_dev, void *y_dev, int i
 /* Mean duration of the SpMV kernel and of the fix-up kernel on the library
  * stream: iters launches of the SpMV kernel back to back between one pair of
  * events, then iters launches of the fix-up between the next pair (a pair of
- * events per launch would add the events' own few microseconds to each).  The
- * kernels keep no state between launches, so repeating one alone is safe; the
- * repeated fix-ups leave y wrong, and a final SpMV puts it right. */
+ * events per launch would add the events' own few microseconds to each).
+ * Repeating one alone is safe: a kernel rewrites its carries, and windowed and
+ * stream tiles leave every partial-sum slot empty again; the repeated fix-ups
+ * leave y wrong, and a final SpMV puts it right. */
 SpB_Info vnec_time_kernels_ext(vnec_plan plan, const void *x_dev, void *y_dev, int iters,
                                double *ms_main, double *ms_fixup)
 {
@@ -1299,15 +1300,16 @@ SpB_Info vnec_time_kernels_ext(vnec_plan plan, const void *x_dev, void *y_dev, i
     vnec_merge_args m;
     /* a relabelled plan's kernels read the permuted x, which the SpMV just
      * before the timed launches leaves in the plan's scratch */
-    fill_args(plan, plan->cperm ? plan->xperm : x_dev, y_dev, &m);
+    const void *xk = plan->cperm ? plan->xperm : x_dev;
+    fill_args(plan, xk, y_dev, &m);
     SpB_Info rc = vnec_plan_run(plan, x_dev, y_dev);
     float a = 0.f, b = 0.f;
     if (rc == SpB_SUCCESS) rc = vnec_hip_ok(hipEventRecord(ev[0], s), "record");
     for (int i = 0; rc == SpB_SUCCESS && i < iters; i++)
-        rc = launch_main(plan, &m, x_dev, y_dev, s);
+        rc = launch_main(plan, &m, xk, y_dev, s);
     if (rc == SpB_SUCCESS) rc = vnec_hip_ok(hipEventRecord(ev[1], s), "record");
     for (int i = 0; rc == SpB_SUCCESS && i < iters; i++)
-        rc = launch_fixup(plan, x_dev, y_dev, s);
+        rc = launch_fixup(plan, xk, y_dev, s);
     if (rc == SpB_SUCCESS) rc = vnec_hip_ok(hipEventRecord(ev[2], s), "record");
     if (rc == SpB_SUCCESS) rc = vnec_hip_ok(hipEventSynchronize(ev[2]), "sync");
     if (rc == SpB_SUCCESS) rc = vnec_hip_ok(hipEventElapsedTime(&a, ev[0], ev[1]), "elapsed");
