@@ -30,6 +30,24 @@ def _windowed(p):
     return bool(spb.L.load().vnec_plan_windowed(p.h))
 
 
+def _chosen(A, variant, ipt, lanes=64):
+    """The plan the library makes of a shape it has chosen itself."""
+    f = spb.L.load().vnec_plan_build_chosen
+    f.argtypes = [spb.C.c_void_p] * 3
+    p = spb.Plan.__new__(spb.Plan)
+    p.A, p.h = A, spb.C.c_void_p()
+    t = spb.L.Tuning(spb.VNEC_VAR[variant], ipt, lanes, spb.VNEC_ENC["fp64"], 1, -1)
+    spb.L.check(f(spb.C.byref(p.h), A.h, spb.C.byref(t)), "vnec_plan_build_chosen")
+    return p
+
+
+def _items(p, m):
+    """Nonzeros per thread of a windowed plan, from its tiles: each holds up to
+    512 of these, rows weighing an eighth."""
+    per = (m.nnz + m.nrows / 8) / p.info().ntiles / 512
+    return next(i for i in (4, 8, 16) if per <= i)
+
+
 def _rows(lens, ncols, seed, cols=None):
     """CSR of the given row lengths; columns random, ascending and distinct
     within a row unless given."""
@@ -99,10 +117,11 @@ MATRICES = {
     "repeated_descending": _repeated_descending,
     "ipt8": lambda: g.powerlaw(60013, 2.2, 3, 20000, seed=9),   # 4096-item tiles, long rows
     "ipt16": lambda: g.rmat(17, 12, seed=10),                   # 8192-item tiles
-    "short_rows": lambda: g.uniform(393241, 3, seed=11),        # as many row sums as window entries
-    "lds_limit": _lds_limit,                                    # 8192-item tiles would not leave room for two
+    "short_rows": lambda: g.uniform(393241, 3, seed=11),        # a row end every two or three nonzeros
+    "lds_limit": _lds_limit,                                    # 8192-item tiles of FP64 leave no room for two
     "dense_row": lambda: g.skew(13, 80, 2, 8000, seed=12),
 }
+ITEMS = {"cut_rows": (4, 4), "ipt8": (8, 8), "ipt16": (16, 16), "short_rows": (4, 4), "lds_limit": (8, 16)}  # FP64, FP32
 
 
 def _check(m, y, enc, ref=None):
@@ -125,6 +144,8 @@ def test_windowed_plan_matches_oracle_and_general_plan(name, enc):
     if p.info().variant == "G":
         pytest.fail("a pattern matrix: not what this test is for")
     assert _windowed(p), p.info()
+    if name in ITEMS:
+        assert _items(p, m) == ITEMS[name][enc == "fp32"]
     q = spb.Plan(A, "L", 7, encoding=enc, grid=-1)  # a named shape keeps its kernel
     assert not _windowed(q)
     dx = spb.DeviceArray.from_array(m.x.astype(dt))
@@ -199,8 +220,8 @@ def test_reference_entries_run_windowed_tiles(kind):
 
 
 def test_window_relabelled_columns_beyond_the_training_sizes():
-    """Above 2^24 nonzeros and 2 MiB of x the learned mode may relabel the
-    columns of windowed tiles hot-first: the same sums either way."""
+    """Above 2^24 nonzeros and 2 MiB of x the learned mode measures windowed
+    tiles over relabelled columns too: the sums are right whichever it keeps."""
     m = g.uniform(2_100_011, 8, seed=15)
     A = spb.Matrix.from_csr(m.nrows, m.ncols, m.ptr, m.col, m.val)
     assert m.nnz > 1 << 24
@@ -214,16 +235,35 @@ def test_window_relabelled_columns_beyond_the_training_sizes():
     p.free()
 
 
+@pytest.mark.parametrize("m", [g.rmat(12, 8, seed=19), g.rmat(17, 12, seed=10)], ids=["4_a_thread", "16_a_thread"])
+def test_windowed_tiles_over_relabelled_columns(m):
+    """Hot-first relabelled columns and a permuted x: the plain plan's bits,
+    direct and replayed."""
+    A = spb.Matrix.from_csr(m.nrows, m.ncols, m.ptr, m.col, m.val)
+    plain, rel = _chosen(A, "L", 7), _chosen(A, "L", 7, spb.LANES_RELABEL)
+    assert _windowed(plain) and _windowed(rel)
+    assert rel.info().lanes & spb.LANES_RELABEL and not plain.info().lanes & spb.LANES_RELABEL
+    dx, ys = spb.DeviceArray.from_array(m.x), []
+    for run in (plain.spmv_dev, rel.spmv_dev, rel.spmv_graph, rel.spmv_graph):
+        dy = spb.DeviceArray.from_array(np.full(m.nrows, np.nan))
+        run(dx.ptr, dy.ptr)
+        ys.append(dy.to_array(np.float64, m.nrows))
+    ok, worst = _check(m, ys[0], "fp64")
+    assert ok, worst
+    for y in ys[1:]:
+        assert np.array_equal(y.view(np.uint64), ys[0].view(np.uint64))
+
+
 @pytest.mark.parametrize("n,hb,windowed", [(29999, 10, True), (30000, 10, False), (14425, 9, False)])
 def test_short_pattern_matrices_run_windowed_tiles(n, hb, windowed):
     """Pattern matrices below 30000 rows of at least 20 entries: windowed tiles
-    under the learned mode's pick, pattern slices where they are named."""
+    where the library has chosen pattern slices, pattern slices where they are
+    named."""
     m = g.banded(n, hb, seed=17)
     A = spb.Matrix.from_csr(m.nrows, m.ncols, m.ptr, m.col, m.val)
-    p, q = spb.Plan(A, "learned"), spb.Plan(A, "G")
-    if p.info().variant == "G":
-        assert _windowed(p) == (windowed and m.nnz >= 20 * n)
-    assert not _windowed(q)
+    p, q = _chosen(A, "G", 8), spb.Plan(A, "G")
+    assert p.info().variant == q.info().variant == "G"
+    assert _windowed(p) == windowed and not _windowed(q)
     dx = spb.DeviceArray.from_array(m.x)
     for plan in (p, q):
         dy = spb.DeviceArray.from_array(np.full(m.nrows, np.nan))
