@@ -194,7 +194,9 @@ def _abs_rows(ptr, col, val, x):
 
 def selector_eval(spb, n):
     """Learned selector vs the plain kernel, the reference dispatch and the
-    exhaustive autotuner, live, on n held-out selector matrices."""
+    exhaustive autotuner, live, on n held-out selector matrices: the named
+    kernels the selector chooses among, and the plan a user of the learned mode
+    gets, which may run windowed tiles in place of the pick."""
     from concurrent.futures import ThreadPoolExecutor
 
     from vnec_amd.selector import specs
@@ -211,19 +213,22 @@ def selector_eval(spb, n):
         learned = spb.select(A, "learned")
         ref = spb.select(A, "reference")
         rule = spb.select(A, "rule")
+        plain = spb.candidates()[PLAIN_CANDIDATE]
         ys = []
-        for c in (learned, PLAIN_CANDIDATE):
-            ci = spb.candidates()[c]
-            p = spb.Plan(A, ci.variant, ci.ipt, grid=ci.grid)
-            xv, yv = spb.Vector.from_array(m.x), spb.Vector(m.nrows)
-            p.spmv(yv, xv)
-            ys.append(yv.to_array())
+        dx, dy = spb.DeviceArray.from_array(m.x), spb.DeviceArray(8 * m.nrows)
+        for p in (spb.Plan(A, "learned"), spb.Plan(A, plain.variant, plain.ipt, grid=plain.grid)):
+            if not ys:
+                t_plan = min(p.time(dx.ptr, dy.ptr, 20) for _ in range(3))
+            p.spmv_dev(dx.ptr, dy.ptr)
+            ys.append(dy.to_array(np.float64, m.nrows))
             p.free()
+        dx.free()
+        dy.free()
         ax = _abs_rows(m.ptr, m.col, m.val, m.x)
         worst = max(worst, float((np.abs(ys[0] - ys[1]) / np.where(ax > 0, ax, 1.0)).max()))
-        rows.append((t[best], t[learned], t[PLAIN_CANDIDATE], t[ref], t[rule]))
+        rows.append((t[best], t[learned], t[PLAIN_CANDIDATE], t[ref], t[rule], t_plan))
         log(f"selector [{i}] {specs.spec(i)['family']:9s} nnz {m.nnz:>9d} best {best:2d} "
-            f"learned {learned:2d} ({t[learned] / t[best]:.3f}x of best)")
+            f"learned {learned:2d} ({t[learned] / t[best]:.3f}x of best), its plan {t_plan / t[best]:.3f}x")
         A.free()
     pool.shutdown()
     r = np.array(rows)
@@ -232,6 +237,8 @@ def selector_eval(spb, n):
             "sample": (f"held-out selector matrices {idx[0]}..{max(idx)} (every 8th of 200: "
                        "R-MAT, banded, block-diagonal, uniform, power-law), timed live with "
                        "hipGraph replay; plain = merge-path CSR kernel, 7 items/thread, persistent"),
+            "learned_plan_vs_plain_speedup_geomean": round(geo(r[:, 2], r[:, 5]), 4),
+            "learned_plan_vs_plain_speedup_aggregate": round(float(r[:, 2].sum() / r[:, 5].sum()), 4),
             "learned_vs_plain_speedup_geomean": round(geo(r[:, 2], r[:, 1]), 4),
             "learned_vs_plain_speedup_aggregate": round(float(r[:, 2].sum() / r[:, 1].sum()), 4),
             "learned_vs_reference_dispatch_speedup_geomean": round(geo(r[:, 3], r[:, 1]), 4),
@@ -241,15 +248,16 @@ def selector_eval(spb, n):
             "max_rel_row_diff_learned_vs_plain": worst}
 
 
-def selection_label(spb, A, mode, info, k):
-    """How the plan was chosen: forced, the MLP's own pick, or the MLP's pick
-    refined by timing its neighbours (beyond the model's training sizes)."""
+def selection_label(spb, A, mode, info, k, windowed=False):
+    """How the plan was chosen: forced, the MLP's own pick (as the kernel it
+    names or as windowed tiles), or the MLP's pick refined by timing its
+    neighbours (beyond the model's training sizes)."""
     if mode is None:
         return "forced"
     if mode == "rule" and info.variant == "G":
         return "rule (pattern rule)"
     if mode != "learned" or k > 1:
-        return mode
+        return mode + ((", windowed tiles" if k == 1 else ", stream tiles") if windowed else "")
     c = spb.candidates()[spb.select(A, "learned")]
     # persistent picks report their workgroup count; per-tile-carry picks (-1)
     # run the strided launch (-2) by themselves once the tiles fill the GPU
@@ -257,6 +265,9 @@ def selection_label(spb, A, mode, info, k):
     flags = info.lanes if info.variant in ("L", "C") and info.lanes != 64 else 0
     extra = ((" 512-thread tiles" if flags & 1024 else "") + (" gathers issued together" if flags & 2048 else "")
              + (" relabelled columns" if flags & 1 else ""))
+    if windowed:
+        over = " over relabelled columns" if flags & 1 else ""
+        return f"learned (MLP pick {c.variant}{c.ipt}, run as windowed tiles{over})"
     if (c.variant, c.ipt, c.lanes) == (info.variant, info.ipt, info.lanes) and same_grid:
         return f"learned (MLP pick: candidate {c.variant}{c.ipt}{extra})"
     form = f"{info.variant}{info.ipt} grid {info.grid}{extra}"
@@ -340,7 +351,7 @@ def measure(spb, lib, name, args, variant=None, mode=None, steps=None, warmup=No
     rec = {
         "workload": desc, "nrows": m.nrows, "nnz": m.nnz, "nrhs": k,
         "plan": {"variant": info.variant, "ipt": info.ipt, "grid": info.grid, "tiles": info.ntiles, "windowed": windowed,
-                 "selection": selection_label(spb, A, None if variant else mode, info, k)},
+                 "selection": selection_label(spb, A, None if variant else mode, info, k, windowed)},
         "format_bytes": fb, "csr_bytes": B,
         "ms_per_step": round(ms_step, 5),
         "GBps": round(fb / (ms_step / 1e3) / 1e9, 1),

@@ -45,3 +45,11 @@ def test_selection_labels():
     assert b.selection_label(None, None, "rule", g, 1) == "rule (pattern rule)"
     assert b.selection_label(None, None, "autotune", g, 1) == "autotune"
     assert b.selection_label(None, None, "learned", g, 8) == "learned"
+    assert b.selection_label(None, None, "learned", g, 8, True) == "learned, stream tiles"
+    assert b.selection_label(None, None, "autotune", g, 1, True) == "autotune, windowed tiles"
+    pick = SimpleNamespace(variant="L", ipt=7, grid=0, lanes=64)
+    spb = SimpleNamespace(candidates=lambda: [pick], select=lambda A, mode: 0)
+    ran = SimpleNamespace(variant="L", ipt=7, grid=-1, lanes=64)  # windowed plans report grid -1
+    assert b.selection_label(spb, None, "learned", ran, 1, True) == "learned (MLP pick L7, run as windowed tiles)"
+    ran.lanes = 1
+    assert b.selection_label(spb, None, "learned", ran, 1, True).endswith("windowed tiles over relabelled columns)")
