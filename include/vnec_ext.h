@@ -181,8 +181,9 @@ SpB_Info vnec_plan_bytes_ext(vnec_plan plan, int64_t *main_bytes, int64_t *spmv_
 SpB_Info vnec_spmv_ext(vnec_plan plan, SpB_Vector y, const SpB_Vector x);
 /* Same on caller device buffers, asynchronous on the library stream.
  * Device buffers hold doubles, or floats for VNEC_ENC_FP32 plans.  With
- * nrhs >= 4, x and y 16-byte aligned run the faster grouped multi-RHS
- * kernel; 8-byte aligned ones are accepted and run the one-lane kernel. */
+ * several right-hand sides, x and y 16-byte aligned run stream tiles (a
+ * chosen plan) or, with nrhs >= 4, the grouped merge-path kernel; 8-byte
+ * aligned ones are accepted and run the slower one-lane merge-path kernel. */
 SpB_Info vnec_spmv_dev_ext(vnec_plan plan, const void *x_dev, void *y_dev);
 /* Same, replayed from a HIP graph: the plan captures its launch sequence
  * for this (x_dev, y_dev) pair on the first call and replays it after
@@ -194,8 +195,9 @@ SpB_Info vnec_spmv_dev_ext(vnec_plan plan, const void *x_dev, void *y_dev);
 SpB_Info vnec_spmv_graph_ext(vnec_plan plan, const void *x_dev, void *y_dev);
 /* Same with the right-hand sides column-major: X holds nrhs vectors of
  * ncols doubles one after another, Y nrhs vectors of nrows.  The plan
- * interleaves X into scratch of its own (allocated on the first call),
- * runs, and writes Y back column-major; for nrhs = 1 this is
+ * interleaves X into scratch of its own (allocated on the first call) and
+ * runs; stream tiles write Y's columns themselves, the merge-path kernel
+ * into scratch that is then laid out column-major.  For nrhs = 1 this is
  * vnec_spmv_dev_ext. */
 SpB_Info vnec_spmm_colmajor_dev_ext(vnec_plan plan, const void *X_dev, void *Y_dev);
 /* Times `iters` back-to-back SpMVs on the library stream with HIP events

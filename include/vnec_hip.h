@@ -249,7 +249,7 @@ typedef struct {
 } vnec_win_args;
 /* Tile boundaries (coords, 2 (P + 1) ints) every `step` units of nonzeros
  * plus rows row8 / 8 (row8: VNEC_WIN_ROW8 for windowed tiles); a tile holds
- * fewer than step + snap nonzeros.  vnec_hip_win_desc: nec may be NULL. */
+ * at most step + snap nonzeros.  vnec_hip_win_desc: nec may be NULL. */
 int vnec_hip_win_coords(const int32_t *ptr, int64_t nrows, int64_t nnz, int64_t P, int row8, int64_t step, int snap,
                         int32_t *coords, void *stream);
 int vnec_hip_win_desc(const int32_t *ptr, int64_t nrows, const int32_t *coords, int64_t ntiles, const int32_t *nec,

@@ -13,9 +13,12 @@
 // product is one launch.
 //
 // What bounds it: each x row is its own 128-byte line (k = 8 holds half of
-// one), pulled from L2 at about 230 G lines/s; the merge-walking kernel this
-// takes over from in chosen plans reached 135 G with its vector units half
-// busy deciding rows.  Measured on one MI355X, replayed, that kernel at 5 items
+// one).  With x rows in L2 that is the rate of the lines: the 28.7M-nonzero batch,
+// k = 8, makes 30.7M requests from L1 to L2 in 185 us (165 G lines/s; bare gathers
+// reach 145-177), where the merge-walking kernel this takes over from in chosen
+// plans reached 135 G with its vector units half busy deciding rows.  With x
+// beyond one XCD's 4 MiB of L2 it is L2's misses: uniform 4.2M, k = 4, x of 8.4 MB,
+// 4.6M requests of which 2.7M miss, 347 MB in 49.6 us (7.0 TB/s).  Measured on one MI355X, replayed, that kernel at 5 items
 // a thread with its carry fix-up against this one:
 //   batch of 28.7M nonzeros   k = 2 187 -> 157 us, 4 199 -> 170, 8 236 -> 179
 //   uniform 4.2M              k = 4 54 -> 50, 8 73.9 -> 66.7

@@ -2,10 +2,12 @@
 // gather their distinct columns of x into LDS once (one right-hand side).
 //
 // What bounds SpMV over scattered columns here is not HBM but the 128-byte
-// lines that x gathers pull from L2 into L1 (about 230 G lines/s whatever the
-// matrix).  Lines fall with the number of nonzeros whose columns are sorted
-// together, so a tile is as large as its x window fits LDS twice per compute
-// unit: 512 threads x 16 nonzeros.  A tile holds
+// lines that x gathers pull from L2 into L1: a kernel that streams the nonzeros
+// and gathers x once for each, no rows, moves 145-177 G lines/s with x of up to
+// 4 MB, which L2 holds, 99 with x of 8 MB and 61 with 32 MB.  Lines fall with the
+// number of nonzeros whose columns are sorted together, so a tile is as large as
+// its x window fits LDS twice per compute unit: 512 threads x 16 nonzeros.  A
+// tile holds
 //   - its distinct columns, ascending (16 bits each, relative to the first of
 //     every 64): gathered in that order, neighbouring lanes share lines, and
 //     a column used many times in the tile is gathered once;
@@ -23,11 +25,17 @@
 // used before against this kernel, us per replayed SpMV (nonzeros; FP64):
 // R-MAT 18 (3.9M) 25.2 -> 17.8, power-law rows (8.0M) 63.4 -> 52.9, R-MAT 20
 // (16M) 98.4 -> 78.0, 1M x 8 uniform (8.0M) 89.9 -> 63.5, 64 block-diagonal
-// members (27M) 121.5 -> 76.8 (4.5 TB/s on the bytes it must move), 16k x 32
+// members (28.7M) 121.5 -> 76.8 (4.5 TB/s on the bytes it must move), 16k x 32
 // uniform (0.5M) 8.4 -> 4.8, R-MAT 10 (12k) 6.8 -> 3.8.  With the gathers
-// replaced by arithmetic the 27M-nonzero batch takes 62 us and R-MAT 18 11.8:
-// what is left above the stream is the line traffic, largely overlapped by the
-// other workgroup of the compute unit.  A persistent form that loads the next
+// replaced by arithmetic the batch takes 62 us and R-MAT 18 11.8: what is left
+// above the stream is the line traffic, partly overlapped by the other workgroup
+// of the compute unit.  Requests from L1 to L2 and L2 misses by counter: R-MAT 18
+// 1.8M and 0.48M in 18.0 us (101 G lines/s), the batch 8.7M and 2.8M in 80.6 (108),
+// R-MAT 20 with dense rows 11.4M and 3.1M in 88.1 (130), power-law rows 7.9M and
+// 1.3M in 52.6 (150).  So power-law rows and R-MAT 20 run at the rate of the bare
+// gathers for their x; R-MAT 18 and the batch leave a third of it idle along a
+// tile's chain of column list, gathers and walk, of which two workgroups hide each
+// other's only in part.  A persistent form that loads the next
 // tile during the walk (128 registers) was slower (R-MAT 18 21.7, batch 85):
 // its waits cover the row stores of the tile before; tiles of 6144 items, three
 // to a compute unit, lose more lines than they hide latency (R-MAT 18 20.4,
@@ -43,8 +51,8 @@
 
 // ------------------------------------------------------------- builders
 // Tile boundaries: rows and nonzeros merged, eight rows weighing as much as
-// row8 nonzeros, cut every `step` units, so a tile holds at most `step`
-// nonzeros and 8 (step + 1) / row8 rows.  W(r) = ptr[r] + r row8 / 8 is the
+// row8 nonzeros, cut every `step` units, so a tile holds at most `step + snap`
+// nonzeros and 8 (step + 1) / row8 + 1 rows.  W(r) = ptr[r] + r row8 / 8 is the
 // weight before row r; the boundary at weight d lies in the last row with
 // W <= d.  With snap > 0 a boundary fewer than snap nonzeros into a row moves
 // to the row's start.

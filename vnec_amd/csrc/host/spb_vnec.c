@@ -392,8 +392,8 @@ SpB_VNEC_type IRD_VNEC(const SpB_Matrix A, SpB_Type type)
 }
 
 /* ------------------------------------------------------ public plans */
-/* The device plan behind a Build_VNEC_* result runs the matching GPU
- * kernel: VNEC-L a merge-path plan (for FP64 the learned selector's pick
+/* The device plan behind a Build_VNEC_* result has the matching GPU shape,
+ * run as windowed tiles where these apply (spb_window.c): VNEC-L a merge-path plan (for FP64 the learned selector's pick
  * when it is one, else 7 items per thread, persistent for FP64, per-tile
  * carries for FP32; tiles in column order where the column-reuse rule
  * holds), VNEC-D the wave64
@@ -409,9 +409,7 @@ static struct vnec_plan_s *gpu_plan_for(spb_csr *a, plan_kind kind)
     if (fp32) t.variant = VNEC_VAR_L; /* grid -1: one workgroup per tile */
     if (kind == KIND_L) {
         /* merge-path CSR: for FP64 the learned selector's pick when it is a
-         * merge-path plan (CSR-ordered or column-sorted tiles, and beyond the
-         * model's training sizes the fastest of the forms measured around
-         * it); otherwise tiles stored in column order where columns are
+         * merge-path plan (CSR-ordered or column-sorted tiles); otherwise tiles stored in column order where columns are
          * reused (the same algorithm, fewer lines per gather) */
         vnec_tuning sel;
         if (!fp32 && vnec_select_tuning(a, VNEC_SELECT_LEARNED, 1, &sel) == SpB_SUCCESS &&
