@@ -168,6 +168,9 @@ SpB_Info vnec_plan_build_ext(vnec_plan *plan, const SpB_Matrix A, const vnec_tun
 SpB_Info vnec_plan_free_ext(vnec_plan *plan);
 /* Tuning in force, tile count and device bytes held by the plan. */
 SpB_Info vnec_plan_info_ext(vnec_plan plan, vnec_tuning *t, int64_t *ntiles, int64_t *dev_bytes);
+/* 1 when the plan runs windowed tiles (or, with several right-hand sides,
+ * stream tiles) in place of the kernel that its tuning names, else 0. */
+int vnec_plan_windowed(vnec_plan plan);
 /* Bytes the plan's own layout must move per SpMV: every array its kernels
  * read counted once, x read once and y written once (padding slots
  * included, caches ignored).  *main_bytes: the main SpMV kernel alone;

@@ -133,6 +133,7 @@ SIGNATURES = {
     "SpB_Vector_device_ptr_ext": (vp, [vp]),
     "vnec_plan_build_ext": (Info, [C.POINTER(vp), vp, C.POINTER(Tuning)]),
     "vnec_plan_free_ext": (Info, [C.POINTER(vp)]),
+    "vnec_plan_windowed": (C.c_int, [vp]),
     "vnec_plan_info_ext": (Info, [vp, C.POINTER(Tuning), C.POINTER(i64), C.POINTER(i64)]),
     "vnec_spmv_ext": (Info, [vp, vp, vp]),
     "vnec_spmv_dev_ext": (Info, [vp, vp, vp]),

@@ -260,8 +260,6 @@ int vnec_streams_run(const struct vnec_plan_s *p, const void *x_dev, const void 
 /* ldy: 0, or the distance of y's columns when they lie one after another. */
 SpB_Info vnec_streams_launch(const struct vnec_plan_s *p, const void *x_dev, void *y_dev, int64_t ldy, hipStream_t s);
 int64_t vnec_streams_bytes(const struct vnec_plan_s *p);
-/* Whether the plan runs as windowed or stream tiles. */
-int vnec_plan_windowed(vnec_plan plan);
 
 /* ---- autotuner and selector (spb_tune.c) ---- */
 /* Tuning chosen by a selection mode (vnec_select_mode) for FP64 values
